@@ -365,12 +365,9 @@ __global__ void vk_repack_w_kq8(int wdtype, const uint8_t* __restrict__ wq, int 
 // bf16 operand (4 values, K 4c..4c+3 of one group) from a nibble word:
 // pairs j0 and j0 + 1. mask = 0x000F000F and magic = 0x43004300 come in
 // registers, so each half is one v_and_or_b32 (a three-operand instruction
-// cannot take literals on this architecture).
-__device__ __forceinline__ uint32_t q4k_and_or(uint32_t x, uint32_t mask, uint32_t magic) {
-    uint32_t r;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "v"(mask), "v"(magic));
-    return r;
-}
+// cannot take literals on this architecture). Not written as inline asm: the
+// compiler counts no wait states from an asm result to the MFMA that reads it.
+__device__ __forceinline__ uint32_t q4k_and_or(uint32_t x, uint32_t mask, uint32_t magic) { return (x & mask) | magic; }
 __device__ __forceinline__ vk_s16x4 q4k_operand(uint32_t w, int j0, uint32_t mask, uint32_t magic) {
     uint2 r;
     r.x = q4k_and_or(w >> (4 * j0), mask, magic);
@@ -646,6 +643,238 @@ __global__ __launch_bounds__(768) void vk_gemm_q4k(const uint4* __restrict__ afr
     }
 }
 
+
+// ---------------------------------------------------------------------------
+// Matmul for many output tiles: a wave keeps 16 x (16 NS) outputs in registers
+// and walks K in group order, so each group's terms are added as soon as they
+// are formed (the same roundings in the same order as vk_gemm_q4k, without the
+// trip of every term through LDS and the adding waves).
+//
+// Bound: the combine's five VALU operations per output and 16-wide group. With
+// two or more waves resident a SIMD issues a plain f32 multiply or add every 2.3
+// clocks (4.5 with one; DPP, integer and three-operand forms 4.2 always) and a
+// 16x16x16 MFMA every 16, and the two do not overlap: a 16 x 16 tile and group
+// is 20 of the former (46 clocks), one MFMA and the unpacking (~16). So:
+//  * the accumulator input -128 * gsum (see vk_gemm_q4k) depends on the rows
+//    alone: one MFMA serves the wave's NT column tiles;
+//  * (s, gsum) come as 16-byte LDS broadcasts rather than DPP operands, which
+//    would run 8 of the 20 at half rate;
+//  * operands go global -> LDS by direct loads through a three-stage ring, a
+//    stage being 8 groups (Q4_K) or 4 (Q5_K, Q6_K): in both one 16-byte weight
+//    word per lane and column tile.
+// A workgroup is WM x (4 / WM) waves (rows x columns) sharing the stage.
+// Measured (Q4_K, us, vk_gemm_q4k -> this): m 413, n 5632, k 2048 89 -> 55 (116
+// clocks per tile and group -> 71 at 2.2 GHz); m 1500, n 5120, k 1280 251 -> 101;
+// Q6_K 98 -> 60 and 292 -> 107.
+namespace kqt {
+constexpr int WAVES = 4, NS = 3, N_XCD = 8;  // waves per workgroup, ring stages
+constexpr int THREADS = 64 * WAVES;
+template <int FMT>
+struct Fmt {
+    static constexpr int GPS = FMT == 0 ? 8 : 4;       // groups per stage
+    static constexpr int SPS = kq::NG / GPS;           // stages per super-block
+    static constexpr int WSB = FMT == 0 ? 2048 : 4096; // weight bytes per super-block and column tile
+};
+}  // namespace kqt
+
+template <int FMT, int WM, int NT>
+__global__ __launch_bounds__(kqt::THREADS, 2) void vk_gemm_kq_tiled(const uint4* __restrict__ afrag,
+                                                                    const float* __restrict__ ascale, VkQ4kSet set,
+                                                                    int m, int nsb, int m_pad, int tiles_m) {
+    using namespace kqt;
+    typedef Fmt<FMT> F;
+    constexpr int WN = WAVES / WM, CT = WN * NT;             // column tiles per workgroup
+    constexpr int AP = F::GPS / 2, RUNS = F::GPS / 4;        // group pairs / runs of 4 groups per stage
+    // direct loads of a stage, 1 KiB each: A fragments, weight words, (d_eff,
+    // m_eff) pairs (two column tiles each), (s, gsum) pairs
+    constexpr int LA = WM * AP, LW = CT, LD = (CT + 1) / 2, LS = WM == 2 ? RUNS : 1;
+    constexpr int LT = LA + LW + LD + LS, LP = (LT + WAVES - 1) / WAVES;
+    constexpr int STAGE = LT * 1024;
+    __shared__ __align__(16) uint8_t ring[NS][STAGE];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / WN, wn = wave % WN;
+
+    // workgroup -> (column block, row block), column-major so that the row
+    // blocks of one column block share its weights in one XCD's L2
+    const int tiles = (int)gridDim.x, L0 = blockIdx.x, per_xcd = tiles / N_XCD;
+    const int t = per_xcd * N_XCD == tiles ? (L0 % N_XCD) * per_xcd + L0 / N_XCD : L0;
+    const int bx = t / tiles_m, mt0 = (t - bx * tiles_m) * WM;
+    const int li = (set.count > 2 && bx >= set.tile0[2]) ? 2 : (set.count > 1 && bx >= set.tile0[1]) ? 1 : 0;
+    const VkQ4kLin L = li == 2 ? set.l[2] : li == 1 ? set.l[1] : set.l[0];
+    const int nt0 = (bx - (li == 2 ? set.tile0[2] : li == 1 ? set.tile0[1] : 0)) * CT;
+    const int nt_last = ((L.n + 15) >> 4) - 1, mt_last = (m_pad >> 4) - 1;
+
+    // this wave's loads: per-lane source, bytes per stage (W: per super-block,
+    // its stages 16 bytes apart), LDS destination. Tiles past the edge re-read
+    // the last one (in bounds, never stored); loads past LT repeat the last.
+    const char* src[LP];
+    size_t adv[LP];
+    bool is_w[LP];
+    uint32_t dst[LP];
+    const uint32_t base = __builtin_amdgcn_readfirstlane(vk_lds_addr(&ring[0][0]));
+#pragma unroll
+    for (int i = 0; i < LP; ++i) {
+        const int q = min(wave + WAVES * i, LT - 1);
+        dst[i] = base + q * 1024;
+        is_w[i] = false;
+        if (q < LA) {
+            const int mt = min(mt0 + q / AP, mt_last);
+            src[i] = reinterpret_cast<const char*>(afrag) + (((size_t)mt * nsb * 8 + q % AP) * 64 + lane) * 16;
+            adv[i] = AP * 1024;
+        } else if (q < LA + LW) {
+            const int nt = min(nt0 + (q - LA), nt_last);
+            src[i] = reinterpret_cast<const char*>(L.wq4) + (size_t)nt * nsb * F::WSB + lane * (F::WSB / 64);
+            adv[i] = F::WSB;
+            is_w[i] = true;
+        } else if (q < LA + LW + LD) {
+            // 32 lanes per column tile: 512 bytes of a stage
+            const int nt = min(nt0 + 2 * (q - LA - LW) + (lane >> 5), nt_last);
+            src[i] = reinterpret_cast<const char*>(L.wdm) + (size_t)nt * nsb * F::SPS * 512 + (lane & 31) * 16;
+            adv[i] = 512;
+        } else {
+            // rows of 32 bytes (4 groups); WM = 2: one run of 32 rows per load,
+            // WM = 1: 16 rows of one or (Q4_K) two runs
+            const int r = WM == 2 ? lane >> 1 : (lane >> 1) & 15;
+            const int run = WM == 2 ? q - LA - LW - LD : (RUNS == 2 ? lane >> 5 : 0);
+            const int row = min(mt0 * 16 + r, m_pad - 1);
+            src[i] = reinterpret_cast<const char*>(ascale) + ((size_t)run * m_pad + row) * 32 + (lane & 1) * 16;
+            adv[i] = (size_t)RUNS * m_pad * 32;
+        }
+    }
+    auto issue = [&](int s, int buf) {
+#pragma unroll
+        for (int i = 0; i < LP; ++i) {
+            const size_t o = is_w[i] ? (size_t)(s / F::SPS) * adv[i] + (s % F::SPS) * 16 : (size_t)s * adv[i];
+            vk_dma_b128(src[i] + o, dst[i] + buf * STAGE);
+        }
+    };
+
+    uint32_t neg128_bf16, nib_mask, byte_mask, magic;
+    asm volatile("v_mov_b32 %0, 0xc300c300" : "=v"(neg128_bf16));
+    asm volatile("v_mov_b32 %0, 0x000f000f" : "=v"(nib_mask));
+    asm volatile("v_mov_b32 %0, 0x00ff00ff" : "=v"(byte_mask));
+    asm volatile("v_mov_b32 %0, 0x43004300" : "=v"(magic));
+    const vk_s16x4 neg128 = __builtin_bit_cast(vk_s16x4, make_uint2(neg128_bf16, neg128_bf16));
+    vk_f32x4 acc[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[j] = (vk_f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+
+    // Four groups of a stage at a time (a run: two fragment pairs, one run of
+    // (s, gsum) pairs). The order is pinned: the run's MFMAs back to back, the
+    // next run's LDS reads, then the run's arithmetic, so neither the matrix
+    // core's nor the LDS latency is waited for with one wave on a SIMD.
+    struct Run {
+        uint4 a[2];        // fragments of the two pairs
+        float4 sg[4][2];   // per row: (s, gsum) of groups 0, 1 and of groups 2, 3
+        float4 dm[NT][2];  // per pair: (d_eff, m_eff) of its two groups
+    };
+    auto compute = [&](int buf) {
+        const uint8_t* st = &ring[buf][0];
+        uint4 wv[NT];
+#pragma unroll
+        for (int j = 0; j < NT; ++j) wv[j] = reinterpret_cast<const uint4*>(st + (LA + wn * NT + j) * 1024)[lane];
+        auto read = [&](int run) {
+            Run o;
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+                o.a[p] = reinterpret_cast<const uint4*>(st + (wm * AP + 2 * run + p) * 1024)[lane];
+            const uint8_t* sp = st + (LA + LW + LD) * 1024 + (WM == 2 ? run * 1024 + wm * 512 : run * 512) + (lane >> 4) * 128;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int p = 0; p < 2; ++p) o.sg[r][p] = *reinterpret_cast<const float4*>(sp + 32 * r + 16 * p);
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                const uint8_t* dp = st + (LA + LW) * 1024 + (wn * NT + j) * 512 + (lane & 15) * 16;
+                if constexpr (FMT == 0) {  // a pair's two groups are one sub-block
+                    const float4 d = *reinterpret_cast<const float4*>(dp + run * 256);
+                    o.dm[j][0] = make_float4(d.x, d.y, d.x, d.y);
+                    o.dm[j][1] = make_float4(d.z, d.w, d.z, d.w);
+                } else {
+                    o.dm[j][0] = *reinterpret_cast<const float4*>(dp);
+                    o.dm[j][1] = *reinterpret_cast<const float4*>(dp + 256);
+                }
+            }
+            return o;
+        };
+        Run cur = read(0);
+#pragma unroll
+        for (int run = 0; run < RUNS; ++run) {
+            vk_f32x4 isum[4][NT];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const uint4 a4 = cur.a[g >> 1];
+                const vk_s16x4 aop =
+                    __builtin_bit_cast(vk_s16x4, (g & 1) ? make_uint2(a4.z, a4.w) : make_uint2(a4.x, a4.y));
+                const vk_f32x4 off = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+                    aop, neg128, (vk_f32x4){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    vk_s16x4 w;
+                    if constexpr (FMT == 0) {
+                        const int wi = 2 * run + (g >> 1);
+                        const uint32_t x = wi == 0 ? wv[j].x : wi == 1 ? wv[j].y : wi == 2 ? wv[j].z : wv[j].w;
+                        w = q4k_operand(x, 2 * (g & 1), nib_mask, magic);
+                    } else {
+                        w = kq_operand<1>(wv[j], g, nib_mask, byte_mask, magic);
+                    }
+                    isum[g][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(aop, w, off, 0, 0, 0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            Run nxt;
+            if (run + 1 < RUNS) nxt = read(run + 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    const float4 d = cur.dm[j][g >> 1];
+                    const float de = (g & 1) ? d.z : d.x, me = (g & 1) ? d.w : d.y;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float4 sg = cur.sg[r][g >> 1];
+                        const float s = (g & 1) ? sg.z : sg.x, gs = (g & 1) ? sg.w : sg.y;
+                        const float x = de * isum[g][j][r], y = me * gs;
+                        acc[j][r] += s * (x - y);
+                    }
+                }
+            if (run + 1 < RUNS) cur = nxt;
+        }
+    };
+
+    // Stage ring: as vk_gemm_qblock's (loads for stage s + 2 issued once every
+    // wave has passed stage s - 1; LP loads per wave and stage, past the end
+    // the last stage again into a buffer that is not read).
+    const int n_st = nsb * F::SPS, last = n_st - 1;
+    issue(0, 0);
+    issue(min(1, last), 1);
+    int buf = 0, nbuf = 2;
+#pragma unroll 1
+    for (int s = 0; s < n_st; ++s) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LP) : "memory");
+        issue(min(s + 2, last), nbuf);
+        compute(buf);
+        buf = buf == NS - 1 ? 0 : buf + 1;
+        nbuf = nbuf == NS - 1 ? 0 : nbuf + 1;
+    }
+    vk_wait_vm<0>();  // no load may land in LDS after the workgroup has ended
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const int col = (nt0 + wn * NT + j) * 16 + (lane & 15);
+        if (col >= L.n) continue;
+        const float b = L.bias ? L.bias[col] : 0.0f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = (mt0 + wm) * 16 + 4 * (lane >> 4) + r;
+            if (row >= m) continue;
+            const size_t o = (size_t)row * L.n + col;
+            L.out[o] = vk_epi_apply(L.bias ? acc[j][r] + b : acc[j][r], L.epi, o);
+        }
+    }
+}
+
 }  // namespace vk
 
 #include "vk_launch.h"
@@ -716,23 +945,70 @@ hipError_t launch_repack_w_q4k(hipStream_t s, const uint8_t* wq, int n, int n_pa
     return hipGetLastError();
 }
 
+// The tiled kernel with WM x (4 / WM) waves of 16 x (16 NT) outputs.
+template <int FMT, int WM, int NT>
+static hipError_t go_kq_tiled(hipStream_t s, const uint4* afrag, const float* ascale, const VkQ4kLin* lins, int n_lin,
+                              int m, int nsb, int m_pad) {
+    constexpr int CT = kqt::WAVES / WM * NT;
+    VkQ4kSet set{};
+    int cols = 0;
+    for (int i = 0; i < n_lin; ++i) {
+        set.l[i] = lins[i];
+        set.tile0[i] = cols;
+        cols += ((lins[i].n + 15) / 16 + CT - 1) / CT;
+    }
+    set.count = n_lin;
+    const int tiles_m = ((m + 15) / 16 + WM - 1) / WM;
+    if ((size_t)cols * tiles_m > (size_t)INT32_MAX) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((vk_gemm_kq_tiled<FMT, WM, NT>), dim3((unsigned)(cols * tiles_m)), dim3(kqt::THREADS), 0, s, afrag,
+                       ascale, set, m, nsb, m_pad, tiles_m);
+    return hipGetLastError();
+}
+
+// 16 x 16 output tiles in the launch from which the tiled kernel runs, and from
+// which its waves take two column tiles. Below, too few of its waves share a
+// SIMD to cover its per-stage latency (~1 us per 8 groups for a lone wave),
+// where vk_gemm_q4k spreads one tile over 12. Measured, us, vk_gemm_q4k / one
+// column tile / two (m, n, k; Q4_K): 1408 tiles (32, 11264, 2048) 16.8 / 18.4 /
+// 22.3; 1504 (1500, 256, 2048) 17.8 / 19.7 / 22.4; 2048 (256, 2048, 2048) 22.6 /
+// 19.4 / 22.6; 2112 (700, 768, 3072) 32.8 / 33.9 / 36.5; 2016 (1000, 512, 512)
+// 14.2 / 7.5 / 8.8; 3008 (1500, 512, 2048) 31.7 / 26.5 / 28.2; 4000 (32, 32000,
+// 2048) 43.9 / 31.4 / 29.0; 7520 (1500, 1280, 1280) 66.1 / 34.6 / 31.9. Four
+// column tiles (218 registers) measured slower than two on every shape but the
+// last (30.9).
+constexpr size_t kKqTiledFrom = 1800, kKqTwoColumnsFrom = 3500;
+
+template <int FMT>
+static hipError_t go_kq(hipStream_t s, const uint4* afrag, const float* ascale, const VkQ4kLin* lins, int n_lin, int m,
+                        int nsb, int m_pad, int tiles) {
+    const int mt = (m + 15) / 16;
+    const size_t out_tiles = (size_t)tiles * mt;
+    if (out_tiles >= kKqTwoColumnsFrom)
+        return mt == 1 ? go_kq_tiled<FMT, 1, 2>(s, afrag, ascale, lins, n_lin, m, nsb, m_pad)
+                       : go_kq_tiled<FMT, 2, 2>(s, afrag, ascale, lins, n_lin, m, nsb, m_pad);
+    if (out_tiles >= kKqTiledFrom)
+        return mt == 1 ? go_kq_tiled<FMT, 1, 1>(s, afrag, ascale, lins, n_lin, m, nsb, m_pad)
+                       : go_kq_tiled<FMT, 2, 1>(s, afrag, ascale, lins, n_lin, m, nsb, m_pad);
+    VkQ4kSet set{};
+    int t0 = 0;
+    for (int i = 0; i < n_lin; ++i) {
+        set.l[i] = lins[i];
+        set.tile0[i] = t0;
+        t0 += (lins[i].n + 15) / 16;
+    }
+    set.count = n_lin;
+    hipLaunchKernelGGL(vk_gemm_q4k<FMT>, dim3((unsigned)tiles, (unsigned)mt), dim3(768), 0, s, afrag, ascale, set, m,
+                       nsb, m_pad);
+    return hipGetLastError();
+}
+
 hipError_t launch_gemm_q4k(hipStream_t s, const uint4* afrag, const float* ascale, const VkQ4kLin* lins, int n_lin,
                            int m, int nsb, int m_pad, int fmt) {
     if (n_lin < 1 || n_lin > 3 || fmt < 0 || fmt > 1) return hipErrorInvalidValue;
-    VkQ4kSet set{};
     int tiles = 0;
-    for (int i = 0; i < n_lin; ++i) {
-        set.l[i] = lins[i];
-        set.tile0[i] = tiles;
-        tiles += (lins[i].n + 15) / 16;
-    }
-    set.count = n_lin;
-    const dim3 grid((unsigned)tiles, (unsigned)((m + 15) / 16));
-    if (fmt == 0)
-        hipLaunchKernelGGL(vk_gemm_q4k<0>, grid, dim3(768), 0, s, afrag, ascale, set, m, nsb, m_pad);
-    else
-        hipLaunchKernelGGL(vk_gemm_q4k<1>, grid, dim3(768), 0, s, afrag, ascale, set, m, nsb, m_pad);
-    return hipGetLastError();
+    for (int i = 0; i < n_lin; ++i) tiles += (lins[i].n + 15) / 16;
+    return fmt == 0 ? go_kq<0>(s, afrag, ascale, lins, n_lin, m, nsb, m_pad, tiles)
+                    : go_kq<1>(s, afrag, ascale, lins, n_lin, m, nsb, m_pad, tiles);
 }
 
 }  // namespace vk
