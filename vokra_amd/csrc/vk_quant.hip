@@ -662,6 +662,177 @@ __global__ __launch_bounds__(gemm::THREADS, 2) void vk_gemm_qblock(
     }
 }
 
+// ---------------------------------------------------------------------------
+// The same block GEMM for grids that leave most SIMDs with one wave or none
+// (short windows, narrow linears): stages of SB quant blocks and smaller wave
+// tiles (16 MT x 16 NT, a workgroup is 2 x 2 waves), same products, same order.
+//
+// Bound: latency. With one wave per SIMD a block of the kernel above takes
+// ~0.27 us (a barrier, the LDS reads, an MFMA and the combine, one after the
+// other), whatever the tile: m 187, n 1280, k 5120 runs 80 workgroups through
+// 160 such steps in 43 us. Here a step is SB blocks: one barrier and one LDS
+// round trip for all of their operands, then their MFMAs back to back, then
+// their combines (the order is pinned), and 32 x 32 workgroup tiles reach four
+// times the SIMDs.
+// Measured (us, vk_gemm_qblock -> 32 x 32 tiles): m 187, n 1280, k 5120 42.1 ->
+// 15.6; m 300, n 1280, k 1280 13.0 -> 7.1; with 64 x 64 tiles, which halve the LDS
+// reads per output: m 1500, n 1280, k 5120 55 -> 45.
+template <bool POW2, int MT, int NT, int SB>
+__global__ __launch_bounds__(gemm::THREADS, 2) void vk_gemm_qblock_deep(
+    const uint4* __restrict__ afrag, const float* __restrict__ ascale, const GemmSet set, int n_lin, int m, int n,
+    int nb, int m_pad, int n_pad, int tiles_m, int tiles_n) {
+    constexpr int WAVES = gemm::WM * gemm::WN;
+    constexpr int AF = 2 * MT * SB, WF = 2 * NT * SB;  // 1 KiB fragments per stage
+    constexpr int APW = AF / WAVES, WPW = WF / WAVES;  // per wave
+    static_assert(APW * WAVES == AF && WPW * WAVES == WF, "whole fragments per wave");
+    static_assert(32 * (MT + NT) * SB == 64 * WAVES, "one scale per thread and stage");
+    constexpr int LOADS = APW + WPW + 1;
+    constexpr int ROWS = 32 * MT, COLS = 32 * NT;
+    __shared__ __align__(16) uint4 lds_a[3][AF * 64];
+    __shared__ __align__(16) uint4 lds_w[3][WF * 64];
+    __shared__ __align__(16) float lds_s[3][64 * WAVES];  // [block][rows, then columns]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 1, wn = wave & 1;
+
+    const int tiles_lin = tiles_m * tiles_n, tiles = tiles_lin * n_lin, L = blockIdx.x, per_xcd = tiles / gemm::N_XCD;
+    const int tt = (per_xcd * gemm::N_XCD == tiles) ? (L % gemm::N_XCD) * per_xcd + L / gemm::N_XCD : L;
+    const int li = tt / tiles_lin, t = tt - li * tiles_lin;
+    const int ntile = t / tiles_m, mtile = t - ntile * tiles_m;
+    const int mt0 = mtile * 2 * MT, nt0 = ntile * 2 * NT;  // first fragment tiles
+    const uint4* __restrict__ wfrag = set.lin[li].wfrag;
+    const float* __restrict__ wscale = set.lin[li].wscale;
+
+    // fragment f of a stage: tile f / SB, block f % SB; wave w moves fragments
+    // w APW .. and w WPW .., the scales one float per thread
+    const int last = nb - 1;
+    // scale sidx of the stage: block sidx / (ROWS + COLS); rows, then columns
+    const int sblk = tid / (ROWS + COLS), sidx = tid % (ROWS + COLS);
+    const float* s_src = sidx < ROWS ? ascale + mt0 * 16 + sidx : wscale + nt0 * 16 + (sidx - ROWS);
+    const int s_stride = sidx < ROWS ? m_pad : n_pad;
+    const uint32_t la = __builtin_amdgcn_readfirstlane(vk_lds_addr(&lds_a[0][wave * APW * 64]));
+    const uint32_t lw = __builtin_amdgcn_readfirstlane(vk_lds_addr(&lds_w[0][wave * WPW * 64]));
+    const uint32_t ls = __builtin_amdgcn_readfirstlane(vk_lds_addr(&lds_s[0][wave * 64]));
+    // blocks past the last re-read it (in bounds, not used)
+    auto issue = [&](int st, int buf) {
+        const int b0 = st * SB;
+#pragma unroll
+        for (int q = 0; q < APW; ++q) {
+            const int f = wave * APW + q;
+            vk_dma_b128(afrag + ((size_t)(mt0 + f / SB) * nb + min(b0 + f % SB, last)) * 64 + lane,
+                        la + buf * (AF * 1024) + q * 1024);
+        }
+#pragma unroll
+        for (int q = 0; q < WPW; ++q) {
+            const int f = wave * WPW + q;
+            vk_dma_b128(wfrag + ((size_t)(nt0 + f / SB) * nb + min(b0 + f % SB, last)) * 64 + lane,
+                        lw + buf * (WF * 1024) + q * 1024);
+        }
+        vk_dma_b32(s_src + (size_t)min(b0 + sblk, last) * s_stride, ls + buf * (64 * WAVES * 4));
+    };
+    vk_f32x4 acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = (vk_f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+    const vk_f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    // cnt: blocks of this stage (SB except in the last one)
+    auto compute = [&](int buf, int cnt) __attribute__((always_inline)) {
+        vk_bf16x8 af[SB][MT], wf[SB][NT];
+        float4 sa[SB][MT];
+        float dw[SB][NT];
+#pragma unroll
+        for (int u = 0; u < SB; ++u) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+                af[u][i] = __builtin_bit_cast(vk_bf16x8, lds_a[buf][((wm * MT + i) * SB + u) * 64 + lane]);
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+                wf[u][j] = __builtin_bit_cast(vk_bf16x8, lds_w[buf][((wn * NT + j) * SB + u) * 64 + lane]);
+        }
+#pragma unroll
+        for (int u = 0; u < SB; ++u) {
+            const float* sc = lds_s[buf] + u * (ROWS + COLS);
+            if (!POW2) {
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+                    sa[u][i] = reinterpret_cast<const float4*>(sc + (wm * MT + i) * 16)[lane >> 4];
+            }
+#pragma unroll
+            for (int j = 0; j < NT; ++j) dw[u][j] = sc[ROWS + (wn * NT + j) * 16 + (lane & 15)];
+        }
+        vk_f32x4 p[SB][MT][NT];
+#pragma unroll
+        for (int u = 0; u < SB; ++u)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+                    p[u][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[u][i], wf[u][j], zero, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < SB; ++u) {
+            if (u >= cnt) break;  // uniform
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                const float sr[4] = {sa[u][i].x, sa[u][i].y, sa[u][i].z, sa[u][i].w};
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        acc[i][j][r] = fmaf(POW2 ? dw[u][j] : sr[r] * dw[u][j], p[u][i][j][r], acc[i][j][r]);
+            }
+        }
+    };
+    // the ring of vk_gemm_qblock: stage s + 2 is issued once every wave has
+    // passed stage s - 1, LOADS loads per wave and stage throughout. (Deeper
+    // rings, and the next stage's LDS reads ahead of the combine, measured the
+    // same or slower: the direct loads' and the LDS reads' rates, ~300 clocks a
+    // stage each, are what a step is made of.)
+    const int n_st = (nb + SB - 1) / SB;
+    issue(0, 0);
+    issue(min(1, n_st - 1), 1);
+    int buf = 0, nbuf = 2;
+#pragma unroll 1
+    for (int st = 0; st < n_st - 1; ++st) {
+        vk_wait_vm_barrier<LOADS>();
+        issue(min(st + 2, n_st - 1), nbuf);
+        compute(buf, SB);
+        buf = buf == 2 ? 0 : buf + 1;
+        nbuf = nbuf == 2 ? 0 : nbuf + 1;
+    }
+    vk_wait_vm_barrier<0>();
+    compute(buf, nb - (n_st - 1) * SB);
+
+    const float* bias = set.lin[li].bias;
+    float* out = set.lin[li].out;
+    const VkEpi epi = set.lin[li].epi;
+    const VkSplitOut so = set.lin[li].so;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const int col = (nt0 + wn * NT + j) * 16 + (lane & 15);
+        if (col >= n) continue;
+        const float bv = bias ? bias[col] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = (mt0 + wm * MT + i) * 16 + 4 * (lane >> 4) + r;
+                if (row >= m) continue;
+                const size_t o = (size_t)row * n + col;
+                const float y = vk_epi_apply(bias ? acc[i][j][r] + bv : acc[i][j][r], epi, o);
+                if (so.hi) {  // row-major split (k)
+                    if (vk_f16_overflow(y)) atomicOr(&vk_gemm_range_flag, 1u);
+                    const _Float16 h = (_Float16)y;
+                    so.hi[o] = __builtin_bit_cast(uint16_t, h);
+                    so.lo[o] = __builtin_bit_cast(uint16_t, (_Float16)(y - (float)h));
+                } else {
+                    out[o] = y;
+                }
+            }
+    }
+}
+
 template __global__ void vk_quantize_act_b32<false>(const float*, int, int, int, uint4*, float*, float*);
 template __global__ void vk_quantize_act_b32<true>(const float*, int, int, int, uint4*, float*, float*);
 
@@ -784,6 +955,21 @@ static_assert(GEMM_TM % gemm::TM == 0 && GEMM_TN % gemm::TN == 0, "GEMM padding"
 // 128 x 128 tiles, 64 x 64 tiles win (measured: 120 tiles 26.5 -> 16.6 us,
 // 360 tiles 37.8 -> 35.4 us; 480 tiles 39.5 -> 46.7 us, so those stay).
 constexpr int kGemmSmallTileBelow = 384;  // 128 x 128 tiles per launch
+// Launches of few 16 x 16 output tiles run vk_gemm_qblock_deep (its f32 and
+// split outputs; the fused activation pass stays with the kernel above): 32 x 32
+// workgroup tiles up to kDeepTiles, fewer when K is long, where each extra
+// round of workgroups costs a whole K loop; then, for long K, 64 x 64 tiles
+// while one resident round (3 workgroups on each of 256 CUs) holds them.
+// Measured, us, vk_gemm_qblock / 32 x 32 / 64 x 64 (m, n, k): 960 tiles (187,
+// 1280, 5120) 42.1 / 15.6 / 35.3; 1520 (300, 1280, 1280) 13.0 / 7.1 / 12.8; 3024
+// (1000, 768, 768) 9.1 / 6.8 / 9.8; 3040 (600, 1280, 5120) 43.4 / 28.1 / 35.9;
+// 3840 (187, 5120, 1280) 15.8 / 12.9 / 13.3; 4000 (2000, 512, 2048) 19.7 / 22.0 /
+// 17.8; 4512 (1500, 768, 3072) 31.0 / 32.0 / 27.4; 6080 (300, 5120, 1280) 16.7 /
+// 19.0 / 15.6; 7520 (1500, 1280, 5120) 55 / 90 / 45; 8000 (4000, 512, 2048) 23.3 /
+// 42.4 / 26.3; 12032, 768 groups (1500, 2048, 5632) 79 / 155 / 71; 15040, 940
+// groups (3000, 1280, 5120) 91 / 178 / 111.
+constexpr size_t kDeepTiles = 4200, kDeepTilesLongK = 3200, kDeepWideGroups = 768;
+constexpr int kDeepWideBlocks = 96;  // k >= 3072
 
 hipError_t launch_gemm_qblock_multi(hipStream_t s, bool pow2, const uint4* afrag, const float* ascale,
                                     const VkGemmLin* lins, int n_lin, int m, int m_pad, int n, int n_pad, int nb) {
@@ -797,7 +983,27 @@ hipError_t launch_gemm_qblock_multi(hipStream_t s, bool pow2, const uint4* afrag
     bool qout = lins[0].qo.afrag != nullptr;
     for (int i = 1; i < n_lin; ++i)
         if ((lins[i].qo.afrag != nullptr) != qout) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)(small ? big * 4 : big)), block(gemm::THREADS);
+    const dim3 block(gemm::THREADS);
+    // 16 x 16 output tiles, and 64 x 64 workgroups of them
+    const size_t t16 = (size_t)((m + 15) / 16) * ((n + 15) / 16) * n_lin;
+    const size_t w64 = (size_t)((m + 63) / 64) * ((n + 63) / 64) * n_lin;
+#define VK_GDEEP(P, MT, NT, SB)                                                                                         \
+    do {                                                                                                               \
+        const int tm = (m + 32 * MT - 1) / (32 * MT), tn = (n + 32 * NT - 1) / (32 * NT);                              \
+        hipLaunchKernelGGL((vk_gemm_qblock_deep<P, MT, NT, SB>), dim3((unsigned)(tm * tn * n_lin)), block, 0, s, afrag, \
+                           ascale, set, n_lin, m, n, nb, m_pad, n_pad, tm, tn);                                        \
+        return hipGetLastError();                                                                                      \
+    } while (0)
+    if (!qout && t16 >= 1 && t16 <= (nb >= 64 ? kDeepTilesLongK : kDeepTiles)) {
+        if (pow2) VK_GDEEP(true, 1, 1, 4);
+        VK_GDEEP(false, 1, 1, 4);
+    }
+    if (!qout && t16 >= 1 && nb >= kDeepWideBlocks && w64 <= kDeepWideGroups) {
+        if (pow2) VK_GDEEP(true, 2, 2, 2);
+        VK_GDEEP(false, 2, 2, 2);
+    }
+#undef VK_GDEEP
+    const dim3 grid((unsigned)(small ? big * 4 : big));
 #define VK_GQ(P, W, Q) hipLaunchKernelGGL((vk_gemm_qblock<P, W, Q>), grid, block, 0, s, afrag, ascale, set, n_lin, m, n, \
                                           nb, n, m_pad, n_pad)
     if (pow2) {
