@@ -168,7 +168,7 @@ struct vokra_hip_qweight {
     size_t n = 0, k = 0, n_pad = 0, nb = 0;
     DevBuf frag, scale;  // MFMA-fragment bf16 integers + f32 scales (prefill GEMM)
     bool has_gemv = false;
-    DevBuf gq, gsc;      // compact decode layout (Q4_0 / Q8_0, k % 128 == 0); Q4_K: nibble words + (d, m)
+    DevBuf gq, gsc;      // compact decode layout (block formats, k % 128 == 0); Q4_K: nibble words + (d, m)
     bool kquant = false; // K-quants: one matmul kernel for every m
     int kfmt = 0;        // its weight layout: 0 nibble words (Q4_K), 1 byte words (Q5_K, Q6_K)
 };
@@ -336,7 +336,7 @@ int upload_weight(vokra_hip_ctx* c, int wdtype, size_t n, size_t k, const uint8_
                                    (uint4*)w->frag.p, (float*)w->scale.p),
            "launch(vk_repack_w_b32)");
     const int mode = wd_kv_mode(wdtype);
-    w->has_gemv = (mode == VOKRA_HIP_KV_Q4_0 || mode == VOKRA_HIP_KV_Q8_0) && w->nb % 4 == 0;
+    w->has_gemv = w->nb % 4 == 0;  // Q4_0, Q8_0, and Q5_0 in Q8_0's layout
     if (w->has_gemv) {
         const size_t qbytes = w->n_pad * w->nb * (mode == VOKRA_HIP_KV_Q4_0 ? 16 : 32);
         VK_TRY(w->gq.ensure(qbytes), "hipMalloc(decode weights)");
@@ -2232,7 +2232,7 @@ int vokra_hip_linear_group_create(vokra_hip_ctx_t* c, size_t count, const vokra_
         if (!w || !d_outs[i]) return fail(VOKRA_HIP_ERROR_INVALID_ARGUMENT, "linear_group_create: NULL entry %zu", i);
         if (w->ctx != c)
             return fail(VOKRA_HIP_ERROR_INVALID_ARGUMENT, "linear_group_create: weight %zu belongs to another context", i);
-        if (w->kquant || !w->has_gemv)
+        if (w->kquant || !w->has_gemv || w->wdtype == VOKRA_HIP_W_Q5_0)
             return fail(VOKRA_HIP_ERROR_UNSUPPORTED_OP,
                         "linear_group_create: weight %zu has no decode layout (Q4_0 / Q8_0 with k %% 128 == 0)", i);
         if (w->wdtype != weights[0]->wdtype || w->k != weights[0]->k)

@@ -11,6 +11,10 @@
 //    so ((X >> 4j) & 0x000F000F) | 0x43004300 is the bf16 pair (128 + nib).
 //  * Q8_0: two 1 KiB fragments per (nt, g), lane l holding 8 bytes q + 128 per
 //    block; v_cvt_f32_ubyte turns each into the exact bf16 of q + 128.
+//  * Q5_0 takes Q8_0's layout (its q in -16..15 as a byte) and kernels: 8 bits
+//    for 5.5, but one pass over the weights instead of the block GEMM's bf16
+//    fragments at 16 (m = 24, n = 5120, k = 1280 on the same activations:
+//    13.0 -> 6.7 us; m = 64, n = 1280, k = 5120 42.2 -> 14.0).
 //  * scales: f16 per (row, block) at [nt][g][16][4] (one 8-byte load per lane).
 //
 // The weight offsets (+128 on every element, and the Q4_0 nibble bias 8) are
@@ -46,7 +50,7 @@ __global__ void vk_repack_w_gemv(int mode, const uint8_t* __restrict__ wq, int n
     const size_t rg = gid >> 2;
     const int row = (int)(rg / G), g = (int)(rg % G);
     const int nt = row >> 4, lane = (row & 15) + 16 * c;
-    const int bb = mode == 3 ? 34 : 18;
+    const int bb = mode == 3 ? 34 : (mode == 2 ? 22 : 18);
     uint32_t w[4] = {0, 0, 0, 0}, w2[4] = {0, 0, 0, 0};
     uint16_t sc[4] = {0, 0, 0, 0};
     for (int u = 0; u < gemv::GB; ++u) {
@@ -62,6 +66,17 @@ __global__ void vk_repack_w_gemv(int mode, const uint8_t* __restrict__ wq, int n
                 x |= (b >> 4) << (16 + 4 * j);
             }
             w[u] = x;
+        } else if (mode == 2) {
+            // Q5_0: q = nibble | fifth bit << 4, minus 16, as Q8_0's bytes
+            const uint32_t qh = p[2] | (p[3] << 8) | (p[4] << 16) | ((uint32_t)p[5] << 24);
+            uint32_t v[2] = {0, 0};
+            for (int e = 0; e < 8; ++e) {
+                const int i = 8 * c + e;
+                const uint32_t nib = (i & 1) ? (p[6 + (i >> 1)] >> 4) : (p[6 + (i >> 1)] & 15u);
+                v[e >> 2] |= ((nib | (((qh >> i) & 1u) << 4)) + 112u) << (8 * (e & 3));
+            }
+            if (u < 2) { w[2 * u] = v[0]; w[2 * u + 1] = v[1]; }
+            else { w2[2 * (u - 2)] = v[0]; w2[2 * (u - 2) + 1] = v[1]; }
         } else {
             uint32_t lo = 0, hi = 0;
             for (int j = 0; j < 4; ++j) {
