@@ -34,6 +34,8 @@
 // layout of the second product, so a lane's V^T operand is one 16-byte read.
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
+
 #include "vk_common.h"
 #include "vk_launch.h"
 
@@ -189,30 +191,81 @@ __global__ void vk_split_rows(const float* __restrict__ x, size_t n4, float scal
                        __builtin_bit_cast(uint16_t, l[2]) | ((uint32_t)__builtin_bit_cast(uint16_t, l[3]) << 16));
 }
 
-// Pre-pass: v [B][T][H*HD] f32 -> transposed hi / lo [B][H][HD][T_pad] fp16,
-// zero for t >= T. One workgroup per (64 x 64 tile of (t, c), head, batch).
-__global__ __launch_bounds__(256) void vk_split_vt(const float* __restrict__ v, int t_kv, int t_pad, int h_kv,
-                                                   int hd, uint16_t* __restrict__ vth, uint16_t* __restrict__ vtl) {
-    __shared__ float tile[64][65];
-    const int t0 = blockIdx.x * 64, c0 = (blockIdx.y % (hd / 64)) * 64, h = blockIdx.y / (hd / 64), b = blockIdx.z;
-    const int tid = threadIdx.x;
-    const size_t width = (size_t)h_kv * hd;
+// hi / lo fp16 of 8 f32 (times 1) as two 16-byte words
+__device__ __forceinline__ void split8_words(const float (&x)[8], uint4& hi, uint4& lo) {
+    uint32_t h[4], l[4];
+    bool bad = false;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int r = (tid >> 6) + 4 * i, c = tid & 63;
-        const int t = t0 + r;
-        tile[r][c] = t < t_kv ? v[((size_t)b * t_kv + t) * width + (size_t)h * hd + c0 + c] : 0.0f;
-        if (vk_f16_overflow(tile[r][c])) attn_range_raise();
+    for (int j = 0; j < 4; ++j) {
+        bad |= vk_f16_overflow(x[2 * j]) || vk_f16_overflow(x[2 * j + 1]);
+        _Float16 h0, l0, h1, l1;
+        split_f16(x[2 * j], h0, l0);
+        split_f16(x[2 * j + 1], h1, l1);
+        h[j] = __builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
+        l[j] = __builtin_bit_cast(uint16_t, l0) | ((uint32_t)__builtin_bit_cast(uint16_t, l1) << 16);
+    }
+    if (bad) attn_range_raise();
+    hi = make_uint4(h[0], h[1], h[2], h[3]);
+    lo = make_uint4(l[0], l[1], l[2], l[3]);
+}
+
+// Pre-pass: v [B][T][H*HD] f32 -> transposed hi / lo [B][H][HD][T_pad] fp16,
+// zero for t >= T, one workgroup per (64 x 64 tile of (t, c), head, batch); and,
+// with nk8 > 0, k -> hi / lo fp16 in its own layout (8 elements per thread) by
+// the workgroups in front of those, so that both passes are one launch.
+// Bound: memory. Rows are read as 16-byte vectors where v allows (V4) and
+// eight consecutive lanes write one 128-byte line of V^T, 16 bytes each (they
+// were 4-byte reads and 2-byte writes). t 1500, 20 heads x 64: the two launches
+// 5.7 + 9.4 us -> 8.2 us in one.
+template <bool V4>
+__global__ __launch_bounds__(256) void vk_split_kv(const float* __restrict__ k, size_t nk8, unsigned k_wgs,
+                                                   uint4* __restrict__ kh, uint4* __restrict__ kl,
+                                                   const float* __restrict__ v, int t_kv, int t_pad, int h_kv, int hd,
+                                                   uint16_t* __restrict__ vth, uint16_t* __restrict__ vtl) {
+    __shared__ float tile[64][65];
+    const int tid = threadIdx.x;
+    if (blockIdx.x < k_wgs) {
+        const size_t i = (size_t)blockIdx.x * 256 + tid;
+        if (i >= nk8) return;
+        const float4 u = reinterpret_cast<const float4*>(k)[2 * i], w = reinterpret_cast<const float4*>(k)[2 * i + 1];
+        const float x[8] = {u.x, u.y, u.z, u.w, w.x, w.y, w.z, w.w};
+        uint4 hi, lo;
+        split8_words(x, hi, lo);
+        kh[i] = hi;
+        kl[i] = lo;
+        return;
+    }
+    const unsigned vt = blockIdx.x - k_wgs, tiles_t = t_pad >> 6, cpt = hd >> 6;
+    const int t0 = (vt % tiles_t) * 64;
+    const unsigned hc = vt / tiles_t;  // (batch * h_kv + head) * cpt + column tile
+    const int c0 = (hc % cpt) * 64, h = (hc / cpt) % h_kv;
+    const size_t b = hc / cpt / h_kv, width = (size_t)h_kv * hd;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int idx = tid + 256 * i, r = idx >> 4, c = 4 * (idx & 15), t = t0 + r;
+        float4 x = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (t < t_kv) {
+            const float* src = v + (b * t_kv + t) * width + (size_t)h * hd + c0 + c;
+            if (V4) x = *reinterpret_cast<const float4*>(src);
+            else x = make_float4(src[0], src[1], src[2], src[3]);
+        }
+        tile[r][c] = x.x;
+        tile[r][c + 1] = x.y;
+        tile[r][c + 2] = x.z;
+        tile[r][c + 3] = x.w;
     }
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int c = (tid >> 6) + 4 * i, r = tid & 63;
-        _Float16 hi, lo;
-        split_f16(tile[r][c], hi, lo);
-        const size_t o = (((size_t)b * h_kv + h) * hd + c0 + c) * t_pad + t0 + r;
-        vth[o] = __builtin_bit_cast(uint16_t, hi);
-        vtl[o] = __builtin_bit_cast(uint16_t, lo);
+    for (int i = 0; i < 2; ++i) {
+        const int c = (tid >> 3) + 32 * i, r = 8 * (tid & 7);
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = tile[r + e][c];
+        uint4 hi, lo;
+        split8_words(x, hi, lo);
+        const size_t o = ((b * h_kv + h) * hd + c0 + c) * t_pad + t0 + r;  // t_pad, t0, r: multiples of 8
+        *reinterpret_cast<uint4*>(vth + o) = hi;
+        *reinterpret_cast<uint4*>(vtl + o) = lo;
     }
 }
 
@@ -288,7 +341,10 @@ __global__ __launch_bounds__(256) void vk_split_vt_q7(const float* __restrict__ 
 // ---------------------------------------------------------------------------
 // LOM: the K / V low parts in use: 0 none (fp16 high parts only), 1 fp16
 // (kl, vtl as fp16 arrays), 2 compact (one byte per element, split_q7).
-template <int HD, int LOM, bool ONEQ>
+// SEQ: the key chunks of sp one after the other in this workgroup, each with a
+// softmax of its own, merged as vk_attn_combine merges them: the results of a
+// launch over chunks without its partials, for batches that fill the chip.
+template <int HD, int LOM, bool ONEQ, bool SEQ = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void vk_flash_attn(
     const uint4* __restrict__ qh, const uint4* __restrict__ ql,    // [B][Tq][Hq*HD] fp16, scaled
     const uint4* __restrict__ kh, const uint4* __restrict__ kl,    // [B][Tkv][Hkv*HD] fp16
@@ -297,7 +353,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void v
     const int* __restrict__ kv_index,
     const float* __restrict__ qf, float q_scale,  // qf != null: f32 q, split here (qh / ql unused)
     const VkQOut qo,                              // qo.afrag != null: quantize O (out may be null)
-    const AttnLayout lay) {                       // K / V element strides
+    const AttnLayout lay,                         // K / V element strides
+    const AttnSplit sp) {                         // key chunks (ONEQ: unused)
     using namespace attn;
     constexpr int KS = HD / 32;      // 32-wide K steps of S = K . Q^T
     constexpr int OS = HD / 16;      // 16-row output subtiles of O^T
@@ -312,7 +369,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void v
     __shared__ __align__(16) _Float16 lv[NP][v_tile_halves(HD)];  // V^T tile, hi (/ lo)
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, lq = lane & 15;
-    const int qt = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+    const int qt = blockIdx.x, h = blockIdx.y;
+    const int b = ONEQ || SEQ ? (int)blockIdx.z : (int)blockIdx.z / sp.n_split;
+    const int chunk_i = ONEQ || SEQ ? 0 : (int)blockIdx.z % sp.n_split;
     const int kb = kv_index ? kv_index[b] : b;  // K/V batch of query batch b
     const int hk = h / (hq / hkv);
     const int q_idx = qt * QT + wave * 16 + lq;  // this lane's query
@@ -320,7 +379,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void v
     // only help stage the K/V tiles
     const bool active = !ONEQ || wave == 0;
     const int q_ld = min(q_idx, tq - 1);
-    const size_t qw = (size_t)hq * HD / 8, kw = (size_t)hkv * HD / 8;  // row widths in uint4
+    const size_t qw = (size_t)hq * HD / 8;  // row width in uint4
+
+    // keys this workgroup has to visit: its query tile's key tiles, or chunk
+    // chunk_i of them
+    int kv_end = tkv;
+    if (causal) kv_end = min(tkv, q_off + min(qt * QT + QT, tq));
+    int n_tiles = (kv_end + KT - 1) / KT, kt_first = 0;
+    bool partial = false;
+    if (!ONEQ && !SEQ && sp.n_split > 1) {
+        kt_first = chunk_i * sp.chunk;
+        if (chunk_i > 0 && kt_first >= n_tiles) return;  // uniform: this query tile has fewer chunks
+        partial = n_tiles > sp.chunk;
+        n_tiles = min(n_tiles, kt_first + sp.chunk);
+    }
 
     // this lane's query operand (B of S^T = K . Q^T): hd 32ks + 8g .. +7
     uint4 qa_h[KS], qa_l[KS];
@@ -340,11 +412,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void v
     for (int ks = 0; ks < KS; ++ks)
         asm volatile("" ::"v"(qa_h[ks].x), "v"(qa_h[ks].y), "v"(qa_h[ks].z), "v"(qa_h[ks].w), "v"(qa_l[ks].x),
                      "v"(qa_l[ks].y), "v"(qa_l[ks].z), "v"(qa_l[ks].w));
-
-    // keys this workgroup has to visit
-    int kv_end = tkv;
-    if (causal) kv_end = min(tkv, q_off + min(qt * QT + QT, tq));
-    const int n_tiles = (kv_end + KT - 1) / KT;
 
     // Staged loads of one K / V^T tile. K: the tile's rows start a buffer
     // resource whose extent ends with row t_kv - 1 of this (batch, kv head)
@@ -600,19 +667,105 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void v
     // causal, at or before the workgroup's first query) are a prefix of
     // the sequence: they run in a loop of their own, so the masked case
     // costs nothing there.
-    Stage st = load(0);  // unconditional (clamped) loads keep the stage in registers
+    // SEQ: the chunks merged so far
+    vk_f32x4 o_sum[SEQ ? OS : 1];
+    float m_sum = -INFINITY, l_sum = 0.0f;
+    int chunk_left = sp.chunk;  // tiles of this chunk (SEQ)
+    bool merged = false;
+    auto merge = [&]() __attribute__((always_inline)) {
+        if (!merged) {
+#pragma unroll
+            for (int os = 0; os < (SEQ ? OS : 1); ++os) o_sum[os] = o_acc[os];
+            m_sum = m_run;
+            l_sum = l_run;
+            merged = true;
+        } else {
+            const float mn = fmaxf(m_sum, m_run), mu = mn == -INFINITY ? 0.0f : mn;
+            const float wa = __builtin_amdgcn_exp2f(m_sum - mu), wb = __builtin_amdgcn_exp2f(m_run - mu);
+#pragma unroll
+            for (int os = 0; os < (SEQ ? OS : 1); ++os)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o_sum[os][r] = fmaf(wb, o_acc[os][r], o_sum[os][r] * wa);
+            l_sum = fmaf(wb, l_run, l_sum * wa);
+            m_sum = mn;
+        }
+#pragma unroll
+        for (int os = 0; os < OS; ++os) o_acc[os] = {0.0f, 0.0f, 0.0f, 0.0f};
+        m_run = -INFINITY;
+        l_run = 0.0f;
+        chunk_left = sp.chunk;
+    };
+    Stage st = load(kt_first);  // unconditional (clamped) loads keep the stage in registers
     auto step = [&](int kt, auto mask_tag) __attribute__((always_inline)) {
         stage_in(st);
         st = load(min(kt + 1, n_tiles - 1));
         if (active) tile(kt, mask_tag);
         VK_LDS_BARRIER();
+        if constexpr (SEQ) {
+            if (--chunk_left == 0 || kt + 1 == n_tiles) merge();  // uniform
+        }
     };
     int n_full = min(n_tiles, tkv / KT);
     if (causal) n_full = min(n_full, (q_off + qt * QT + 1) / KT);
-    int kt = 0;
+    int kt = kt_first;
     for (; kt < n_full; ++kt) step(kt, AttnMask<false>{});
     for (; kt < n_tiles; ++kt) step(kt, AttnMask<true>{});
+    if constexpr (SEQ) {
+        finish(o_sum, l_sum > 0.0f ? 1.0f / l_sum : 0.0f);
+        return;
+    }
+    if constexpr (!ONEQ && !SEQ) {
+        if (partial) {  // this chunk's (max, sum) and unscaled O; vk_attn_combine merges the chunks
+            const size_t pid = (((size_t)b * hq + h) * gridDim.x + qt) * sp.n_split + chunk_i;
+            const int row = wave * 16 + lq;
+            float* po = sp.o + (pid * QT + row) * HD;
+#pragma unroll
+            for (int os = 0; os < OS; ++os)
+                *reinterpret_cast<float4*>(po + 16 * os + 4 * g) =
+                    make_float4(o_acc[os][0], o_acc[os][1], o_acc[os][2], o_acc[os][3]);
+            if (g == 0) sp.ml[pid * QT + row] = make_float2(m_run, l_run);
+            return;
+        }
+    }
     if (active) finish(o_acc, l_run > 0.0f ? 1.0f / l_run : 0.0f);
+}
+
+// Merges the chunks of the query tiles that have more than one, in order: with
+// (M, l, O) so far and chunk s, M' = max(M, m_s), O' = 2^(M - M') O + 2^(m_s - M')
+// O_s, l' likewise (base-2 units); out = O / l. HD / 4 lanes per (query, head).
+template <int HD>
+__global__ __launch_bounds__(256) void vk_attn_combine(const AttnSplit sp, float* __restrict__ out, int tq, int tkv,
+                                                       int hq, int causal, int q_off) {
+    using namespace attn;
+    constexpr int LPR = HD / 4, ROWS = 256 / LPR;
+    const int q = blockIdx.x * ROWS + (int)threadIdx.x / LPR, d = 4 * ((int)threadIdx.x % LPR), h = blockIdx.y,
+              b = blockIdx.z;
+    if (q >= tq) return;
+    const int qt = q / QT, n_qt = (tq + QT - 1) / QT;
+    int kv_end = tkv;
+    if (causal) kv_end = min(tkv, q_off + min(qt * QT + QT, tq));
+    const int n_ch = ((kv_end + KT - 1) / KT + sp.chunk - 1) / sp.chunk;
+    if (n_ch <= 1) return;  // written by its one workgroup
+    const size_t r0 = (((size_t)b * hq + h) * n_qt + qt) * sp.n_split * QT + q % QT;
+    float2 ml = sp.ml[r0];
+    float mx = ml.x, l = ml.y;
+    float4 o = *reinterpret_cast<const float4*>(sp.o + r0 * HD + d);
+    for (int s = 1; s < n_ch; ++s) {
+        const size_t r = r0 + (size_t)s * QT;
+        ml = sp.ml[r];
+        const float4 x = *reinterpret_cast<const float4*>(sp.o + r * HD + d);
+        const float mn = fmaxf(mx, ml.x), mu = mn == -INFINITY ? 0.0f : mn;
+        const float wa = __builtin_amdgcn_exp2f(mx - mu), wb = __builtin_amdgcn_exp2f(ml.x - mu);
+        l = fmaf(wb, ml.y, l * wa);
+        o.x = fmaf(wb, x.x, o.x * wa);
+        o.y = fmaf(wb, x.y, o.y * wa);
+        o.z = fmaf(wb, x.z, o.z * wa);
+        o.w = fmaf(wb, x.w, o.w * wa);
+        mx = mn;
+    }
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    *reinterpret_cast<float4*>(out + ((size_t)b * tq + q) * (size_t)hq * HD + (size_t)h * HD + d) =
+        make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
 }
 
 }  // namespace vk
@@ -656,12 +809,25 @@ hipError_t launch_split_rows_q7_heads(hipStream_t s, const float* x, int batch, 
     return hipGetLastError();
 }
 
+hipError_t launch_split_kv(hipStream_t s, const float* k, size_t nk, void* kh, void* kl, const float* v, int batch,
+                           int t_kv, int t_pad, int h_kv, int hd, void* vth, void* vtl) {
+    const size_t nk8 = nk / 8, k_wgs = (nk8 + 255) / 256;
+    const size_t v_wgs = (size_t)(t_pad / 64) * h_kv * (hd / 64) * batch, wgs = k_wgs + v_wgs;
+    if (wgs == 0) return hipSuccess;
+    if (wgs > (size_t)INT32_MAX) return hipErrorInvalidValue;
+    if ((reinterpret_cast<uintptr_t>(v) & 15) == 0)
+        hipLaunchKernelGGL(vk_split_kv<true>, dim3((unsigned)wgs), dim3(256), 0, s, k, nk8, (unsigned)k_wgs, (uint4*)kh,
+                           (uint4*)kl, v, t_kv, t_pad, h_kv, hd, (uint16_t*)vth, (uint16_t*)vtl);
+    else
+        hipLaunchKernelGGL(vk_split_kv<false>, dim3((unsigned)wgs), dim3(256), 0, s, k, nk8, (unsigned)k_wgs, (uint4*)kh,
+                           (uint4*)kl, v, t_kv, t_pad, h_kv, hd, (uint16_t*)vth, (uint16_t*)vtl);
+    return hipGetLastError();
+}
+
 hipError_t launch_split_vt(hipStream_t s, const float* v, int batch, int t_kv, int t_pad, int h_kv, int hd, void* vth,
                            void* vtl) {
     if (batch == 0 || t_pad == 0) return hipSuccess;
-    hipLaunchKernelGGL(vk_split_vt, dim3(t_pad / 64, h_kv * (hd / 64), batch), dim3(256), 0, s, v, t_kv, t_pad, h_kv,
-                       hd, (uint16_t*)vth, (uint16_t*)vtl);
-    return hipGetLastError();
+    return launch_split_kv(s, nullptr, 0, nullptr, nullptr, v, batch, t_kv, t_pad, h_kv, hd, vth, vtl);
 }
 
 AttnLayout attn_layout_rows(int t_kv, int h_kv, int hd, int t_pad) {
@@ -696,6 +862,7 @@ struct FlashArgs {
     float q_scale;
     VkQOut qo;
     AttnLayout lay;
+    AttnSplit sp = {nullptr, nullptr, 1, 0};
 };
 
 // Dynamic LDS that sets a single-query launch's residency. Those launches
@@ -746,7 +913,7 @@ void go_flash(hipStream_t s, dim3 grid, const FlashArgs& a) {
     hipLaunchKernelGGL((vk_flash_attn<HD, LOM, ONEQ>), grid, dim3(256), pad, s, (const uint4*)a.qh,
                        (const uint4*)a.ql, (const uint4*)a.kh, (const uint4*)a.kl, (const uint4*)a.vth,
                        (const uint4*)a.vtl, a.out, a.tq, a.tkv, a.t_pad, a.hq, a.hkv, a.causal, a.q_off, a.kv_index,
-                       a.qf, a.q_scale, a.qo, a.lay);
+                       a.qf, a.q_scale, a.qo, a.lay, a.sp);
 }
 
 template <int HD>
@@ -766,7 +933,7 @@ hipError_t flash_any(hipStream_t s, int hd, int batch, int lo_mode, const FlashA
     // per-lane 32-bit K offsets, in bytes
     if ((size_t)hd * a.t_pad * 2 > 0x7fffffffu || (size_t)attn::KT * a.lay.kt * 2 > 0x7fffffffu)
         return hipErrorInvalidValue;
-    const dim3 grid((a.tq + attn::QT - 1) / attn::QT, a.hq, batch);
+    const dim3 grid((a.tq + attn::QT - 1) / attn::QT, a.hq, batch * a.sp.n_split);
     if (hd == 64)
         go_flash_hd<64>(s, grid, lo_mode, a);
     else
@@ -793,6 +960,78 @@ hipError_t launch_flash_attn_f32q(hipStream_t s, int hd, const float* q, float q
                          causal,  q_off,   kv_index, q,   attn_q_scale(q_scale), qo ? *qo : VkQOut{},
                          lay ? *lay : attn_layout_rows(tkv, hkv, hd, t_pad)};
     return flash_any(s, hd, batch, lo_mode, a);
+}
+
+// Key chunks of one item's attention (t_q >= 2): an item whose (query tile,
+// head) pairs leave most of the chip idle splits its key tiles so that about
+// kSplitTarget workgroups share them, at least two tiles each, merged by
+// vk_attn_combine. Decided by the item's own shape alone, so that an item's
+// result does not depend on the batch around it. Splitting costs the partial
+// results' round trip and one launch (~6 us), so it is taken when it shortens
+// the longest workgroup's loop to 55 % or less: a causal prompt's unequal query
+// tiles, cross-attention with few queries, a few heads.
+// Measured (whole calls, us, before -> after): 1 x 777 causal, 16 / 2 heads x 128 48.4
+// -> 33.3; 1 x 1500, 8 heads x 64 51 -> 38; 16 queries over 1500 keys, 20 heads 51 ->
+// 22; 64 causal after 300, 32 / 8 x 128 29 -> 20; 8 x 1500, 8 heads (in place) 158 -> 163
+constexpr long long kSplitTarget = 480;
+int attn_key_splits(int tq, int tkv, int hq, int causal, int q_off, int* chunk) {
+    *chunk = 0;
+    if (tq < 2 || tkv < 1) return 1;
+    const long long nqt = (tq + attn::QT - 1) / attn::QT;
+    if (nqt * hq > kSplitTarget) return 1;
+    long long total = 0, longest = 0;
+    for (long long qt = 0; qt < nqt; ++qt) {
+        long long end = tkv;
+        if (causal) end = std::min<long long>(tkv, q_off + std::min<long long>((qt + 1) * attn::QT, tq));
+        const long long t = (end + attn::KT - 1) / attn::KT;
+        total += t * hq;
+        longest = std::max(longest, t);
+    }
+    long long c = std::max<long long>(2, (total + kSplitTarget - 1) / kSplitTarget);
+    if (c * 100 > longest * 55) return 1;
+    const long long n = (longest + c - 1) / c;
+    c = (longest + n - 1) / n;  // even chunks of the longest loop
+    *chunk = (int)c;
+    return (int)n;
+}
+
+// Whether a batch's chunks run inside one workgroup per query tile instead
+// (SEQ; head_dim 64, where the merged state fits the registers): from one and a
+// half rounds of two workgroups per CU on, the chip is full without the split.
+bool attn_split_in_place(int hd, int batch, int tq, int hq) {
+    return hd == 64 && (long long)batch * hq * ((tq + attn::QT - 1) / attn::QT) >= 768;
+}
+
+size_t attn_split_rows(int batch, int tq, int hq, int n_split) {
+    return (size_t)batch * hq * ((tq + attn::QT - 1) / attn::QT) * n_split * attn::QT;
+}
+
+hipError_t launch_flash_attn_split(hipStream_t s, int hd, const float* q, float q_scale, const void* kh, const void* kl,
+                                   const void* vth, const void* vtl, float* out, int batch, int tq, int tkv, int t_pad,
+                                   int hq, int hkv, int causal, int q_off, const AttnSplit& sp) {
+    if ((long long)batch * sp.n_split > 65535 || sp.n_split < 2 || sp.chunk < 1) return hipErrorInvalidValue;
+    const bool seq = attn_split_in_place(hd, batch, tq, hq);
+    FlashArgs a = {nullptr, nullptr, kh,     kl,      vth, vtl,
+                   out,     tq,      tkv,    t_pad,   hq,  hkv,
+                   causal,  q_off,   nullptr, q,      attn_q_scale(q_scale), VkQOut{},
+                   attn_layout_rows(tkv, hkv, hd, t_pad)};
+    a.sp = sp;
+    if (seq) {
+        hipLaunchKernelGGL((vk_flash_attn<64, 1, false, true>), dim3((tq + attn::QT - 1) / attn::QT, hq, batch), dim3(256), 0,
+                           s, (const uint4*)a.qh, (const uint4*)a.ql, (const uint4*)a.kh, (const uint4*)a.kl,
+                           (const uint4*)a.vth, (const uint4*)a.vtl, a.out, a.tq, a.tkv, a.t_pad, a.hq, a.hkv, a.causal,
+                           a.q_off, a.kv_index, a.qf, a.q_scale, a.qo, a.lay, a.sp);
+        return hipGetLastError();
+    }
+    hipError_t e = flash_any(s, hd, batch, KV_LO_F16, a);
+    if (e != hipSuccess) return e;
+    if (hd == 64)
+        hipLaunchKernelGGL(vk_attn_combine<64>, dim3((tq + 15) / 16, hq, batch), dim3(256), 0, s, sp, out, tq, tkv, hq,
+                           causal, q_off);
+    else
+        hipLaunchKernelGGL(vk_attn_combine<128>, dim3((tq + 7) / 8, hq, batch), dim3(256), 0, s, sp, out, tq, tkv, hq,
+                           causal, q_off);
+    return hipGetLastError();
 }
 
 // This device's address of this file's fp16-range flag (the host reads and

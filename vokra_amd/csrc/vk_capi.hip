@@ -148,6 +148,7 @@ struct vokra_hip_ctx {
     vokra_hip_qact act;
     // attention workspace: fp16 hi / lo splits of q, k and transposed v
     DevBuf at_qh, at_ql, at_kh, at_kl, at_vh, at_vl;
+    DevBuf at_po, at_pml;  // key-split partials (vk::AttnSplit)
     // front end: window, DFT basis, filter bank (for fe_mels bands), frames,
     // spectrum, power, mel energies, per-block maxima; im2col columns
     DevBuf fe_win, fe_basis, fe_fb, fe_frames, fe_spec, fe_pow, fe_mel, fe_part, cv_col;
@@ -414,8 +415,32 @@ int check_attn(size_t batch, size_t tq, size_t tkv, size_t hq, size_t hkv, size_
     return VOKRA_HIP_OK;
 }
 
+// The key chunks of an attention call over several query rows (n_split = 1:
+// none), its partials' workspace in place. A capture cannot allocate: a call
+// whose partials no earlier call made room for records the undivided launch.
+int attn_split_for(vokra_hip_ctx* c, size_t batch, size_t tq, size_t tkv, size_t hq, size_t hd, int causal,
+                   size_t q_off, vk::AttnSplit* sp) {
+    *sp = vk::AttnSplit{nullptr, nullptr, 1, 0};
+    if (q_off > (size_t)INT32_MAX / 2) return VOKRA_HIP_OK;
+    int chunk = 0;
+    const int n = vk::attn_key_splits((int)tq, (int)tkv, (int)hq, causal ? 1 : 0, (int)q_off, &chunk);
+    if (n <= 1 || batch * n > 65535) return VOKRA_HIP_OK;
+    const bool in_place = vk::attn_split_in_place((int)hd, (int)batch, (int)tq, (int)hq);
+    const size_t rows = in_place ? 0 : vk::attn_split_rows((int)batch, (int)tq, (int)hq, n);
+    if (c->at_po.cap < rows * hd * sizeof(float) || c->at_pml.cap < rows * sizeof(float2)) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        VK_TRY(hipStreamIsCapturing(c->stream, &cs), "hipStreamIsCapturing");
+        if (cs != hipStreamCaptureStatusNone) return VOKRA_HIP_OK;
+        VK_TRY(c->at_po.ensure(rows * hd * sizeof(float)), "hipMalloc(attention partials)");
+        VK_TRY(c->at_pml.ensure(rows * sizeof(float2)), "hipMalloc(attention partials)");
+    }
+    *sp = vk::AttnSplit{(float*)c->at_po.p, (float2*)c->at_pml.p, n, chunk};
+    return VOKRA_HIP_OK;
+}
+
 // With qo (a fused activation pass over the output rows), d_out is still
-// written when keep_out is set or q is unaligned (the pass then runs on it).
+// written when keep_out is set, when q is unaligned or when the keys split
+// (the pass then runs on it).
 int run_attn(vokra_hip_ctx* c, size_t batch, size_t tq, size_t tkv, size_t hq, size_t hkv, size_t hd,
              const float* d_q, const float* d_k, const float* d_v, float scale, int causal, size_t q_off,
              float* d_out, const VkQOut* qo = nullptr, bool keep_out = true) {
@@ -446,10 +471,25 @@ int run_attn(vokra_hip_ctx* c, size_t batch, size_t tq, size_t tkv, size_t hq, s
                                       c->at_vl.p),
                "launch(vk_split_vt_q7)");
     } else {
-        VK_TRY(vk::launch_split_rows(c->stream, d_k, nk, 1.0f, c->at_kh.p, c->at_kl.p), "launch(vk_split_rows k)");
-        VK_TRY(vk::launch_split_vt(c->stream, d_v, (int)batch, (int)tkv, (int)t_pad, (int)hkv, (int)hd, c->at_vh.p,
-                                   c->at_vl.p),
-               "launch(vk_split_vt)");
+        VK_TRY(vk::launch_split_kv(c->stream, d_k, nk, c->at_kh.p, c->at_kl.p, d_v, (int)batch, (int)tkv, (int)t_pad,
+                                   (int)hkv, (int)hd, c->at_vh.p, c->at_vl.p),
+               "launch(vk_split_kv)");
+    }
+    vk::AttnSplit sp;
+    if (q_in_kernel && !q7) {
+        int st = attn_split_for(c, batch, tq, tkv, hq, hd, causal, q_off, &sp);
+        if (st) return st;
+        if (sp.n_split > 1) {
+            VK_TRY(vk::launch_flash_attn_split(c->stream, (int)hd, d_q, scale, c->at_kh.p, c->at_kl.p, c->at_vh.p,
+                                               c->at_vl.p, d_out, (int)batch, (int)tq, (int)tkv, (int)t_pad, (int)hq,
+                                               (int)hkv, causal ? 1 : 0, (int)q_off, sp),
+                   "launch(vk_flash_attn x key splits)");
+            if (qo)
+                VK_TRY(vk::launch_quantize_act_b32(c->stream, qo->pow2 != 0, d_out, (int)(batch * tq), qo->m_pad, qo->k,
+                                                   qo->afrag, qo->ascale, qo->asum),
+                       "launch(vk_quantize_act_b32)");
+            return VOKRA_HIP_OK;
+        }
     }
     if (q_in_kernel) {
         VK_TRY(vk::launch_flash_attn_f32q(c->stream, (int)hd, d_q, scale, c->at_kh.p, c->at_kl.p, c->at_vh.p,
@@ -819,9 +859,21 @@ int attn_quantize_split(vokra_hip_ctx* c, size_t batch, size_t t, size_t h, size
         (reinterpret_cast<uintptr_t>(d_q) & 15))
         return fail(VOKRA_HIP_ERROR_INVALID_ARGUMENT, "attn: split operands need the fused activation pass");
     VK_TRY(set_dev(c), "hipSetDevice");
-    VK_TRY(vk::launch_flash_attn_f32q(c->stream, (int)hd, d_q, scale, kh, kl, vth, vtl, nullptr, (int)batch, (int)t,
-                                      (int)t, (int)t_pad, (int)h, (int)h, 0, 0, nullptr, vk::KV_LO_F16, &qo),
-           "launch(vk_flash_attn)");
+    vk::AttnSplit sp;
+    st = attn_split_for(c, batch, t, t, h, hd, 0, 0, &sp);
+    if (st) return st;
+    if (sp.n_split > 1) {  // as run_attn: the merged rows, then the activation pass
+        VK_TRY(vk::launch_flash_attn_split(c->stream, (int)hd, d_q, scale, kh, kl, vth, vtl, d_out, (int)batch, (int)t,
+                                           (int)t, (int)t_pad, (int)h, (int)h, 0, 0, sp),
+               "launch(vk_flash_attn x key splits)");
+        VK_TRY(vk::launch_quantize_act_b32(c->stream, qo.pow2 != 0, d_out, (int)(batch * t), qo.m_pad, qo.k, qo.afrag,
+                                           qo.ascale, qo.asum),
+               "launch(vk_quantize_act_b32)");
+    } else {
+        VK_TRY(vk::launch_flash_attn_f32q(c->stream, (int)hd, d_q, scale, kh, kl, vth, vtl, nullptr, (int)batch, (int)t,
+                                          (int)t, (int)t_pad, (int)h, (int)h, 0, 0, nullptr, vk::KV_LO_F16, &qo),
+               "launch(vk_flash_attn)");
+    }
     qact_commit(qa, batch * t, act_quant);
     return VOKRA_HIP_OK;
 }
@@ -1732,7 +1784,7 @@ void vokra_hip_destroy(vokra_hip_ctx_t* c) {
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
     for (DevBuf* b : {&c->in0, &c->in1, &c->in2, &c->out0, &c->act.frag, &c->act.scale, &c->act.gsum, &c->at_qh,
-                      &c->at_ql, &c->at_kh, &c->at_kl, &c->at_vh, &c->at_vl, &c->fe_win, &c->fe_basis, &c->fe_fb,
+                      &c->at_ql, &c->at_kh, &c->at_kl, &c->at_vh, &c->at_vl, &c->at_po, &c->at_pml, &c->fe_win, &c->fe_basis, &c->fe_fb,
                       &c->fe_frames, &c->fe_spec, &c->fe_pow, &c->fe_mel, &c->fe_part, &c->cv_col, &c->lg_part,
                       &c->rope_theta, &c->rope_pos})
         b->release();

@@ -141,6 +141,32 @@ hipError_t launch_swiglu_quantize_g16(hipStream_t s, const float* g, const float
 }  // namespace vk
 
 namespace vk {
+// The conv stem (vk_stem.hip): weights as scaled fp16 hi / lo [out][3][channels]
+// (channels padded to stem_channels), and a batch's workspaces: hi / lo rows of
+// the log-mel [clip][n_frames + 2][stem_channels(n_mels)] and of the first
+// convolution's output [clip][n_frames + 2][d], and stem_scalars(batch) floats.
+struct StemW {
+    const void *w1hi, *w1lo, *w2hi, *w2lo;
+    int e1, e2;  // their scales' exponents
+    const float *b1, *b2, *pos;
+    float l1max, bmax;  // largest row L1 norm of conv1's weights, largest |conv1 bias|
+};
+struct StemBufs {
+    void *ahi, *alo, *hhi, *hlo;
+    float* scal;
+};
+inline int stem_channels(int c) { return (c + 31) / 32 * 32; }
+size_t stem_scalars(size_t batch);
+int stem_weight_exponent(const float* w, size_t n);
+hipError_t launch_stem_pack(hipStream_t s, const float* w, int out, int c, int cp, int e, void* hi, void* lo);
+hipError_t launch_stem(hipStream_t s, const float* mel, int batch, int nm, int nf, int nc, int d, const StemW& w,
+                       const StemBufs& b, float* out);
+}  // namespace vk
+
+namespace vk {
+// k (nk elements, a multiple of 8) -> hi / lo fp16 in its layout, and v -> V^T hi / lo, in one launch.
+hipError_t launch_split_kv(hipStream_t s, const float* k, size_t nk, void* kh, void* kl, const float* v, int batch,
+                           int t_kv, int t_pad, int h_kv, int hd, void* vth, void* vtl);
 hipError_t launch_split_rows(hipStream_t s, const float* x, size_t n, float scale, void* hi, void* lo);
 hipError_t launch_split_vt(hipStream_t s, const float* v, int batch, int t_kv, int t_pad, int h_kv, int hd, void* vth,
                            void* vtl);
@@ -152,6 +178,14 @@ hipError_t launch_split_vt_q7(hipStream_t s, const float* v, int batch, int t_kv
 // x [B][T][H*hd] -> hi / lo [B][H][T][hd] (the attn_layout_heads K form)
 hipError_t launch_split_rows_q7_heads(hipStream_t s, const float* x, int batch, int t, int h, int hd, float scale,
                                       void* hi, void* lo);
+// Key chunks of an attention launch (attn_key_splits): n_split > 1 chunks of
+// `chunk` 64-key tiles per query tile. Row ((batch, head, query tile), chunk,
+// query of the tile): its unscaled O (head_dim floats) and (max, sum).
+struct AttnSplit {
+    float* o;
+    float2* ml;
+    int n_split, chunk;
+};
 // Element strides of a flash launch's K / V operands: K element (b, t, h, d)
 // at b * kb + h * kh + t * kt + d; V^T element (b, h, d, t) at
 // (b * h_kv + h) * hd * t_pad + (t / 64) * vtile + d * vd + t % 64.
@@ -182,6 +216,15 @@ hipError_t launch_flash_attn(hipStream_t s, int hd, const void* qh, const void* 
 // as launch_split_rows would. With qo, the
 // kernel also quantizes O (rows b * tq + i, width hq * hd) into qo's
 // activation fragments, and out may be null.
+// How many chunks (1: none) the keys of one item's attention split into, and
+// the chunks' length in 64-key tiles; the workspace rows of such a launch.
+int attn_key_splits(int tq, int tkv, int hq, int causal, int q_off, int* chunk);
+size_t attn_split_rows(int batch, int tq, int hq, int n_split);
+bool attn_split_in_place(int hd, int batch, int tq, int hq);  // no partials: rows not needed
+// The flash launch over the chunks (f32 q, fp16 low parts) and their merge.
+hipError_t launch_flash_attn_split(hipStream_t s, int hd, const float* q, float q_scale, const void* kh, const void* kl,
+                                   const void* vth, const void* vtl, float* out, int batch, int tq, int tkv, int t_pad,
+                                   int hq, int hkv, int causal, int q_off, const AttnSplit& sp);
 hipError_t launch_flash_attn_f32q(hipStream_t s, int hd, const float* q, float q_scale, const void* kh, const void* kl,
                                   const void* vth, const void* vtl, float* out, int batch, int tq, int tkv, int t_pad,
                                   int hq, int hkv, int causal, int q_off, const int* kv_index = nullptr,
