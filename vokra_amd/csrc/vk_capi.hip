@@ -149,9 +149,9 @@ struct vokra_hip_ctx {
     // attention workspace: fp16 hi / lo splits of q, k and transposed v
     DevBuf at_qh, at_ql, at_kh, at_kl, at_vh, at_vl;
     DevBuf at_po, at_pml;  // key-split partials (vk::AttnSplit)
-    // front end: window, DFT basis, filter bank (for fe_mels bands), frames,
-    // spectrum, power, mel energies, per-block maxima; im2col columns
-    DevBuf fe_win, fe_basis, fe_fb, fe_frames, fe_spec, fe_pow, fe_mel, fe_part, cv_col;
+    // front end: window, twiddles, filter bank (for fe_mels bands), per-block
+    // maxima; im2col columns
+    DevBuf fe_win, fe_tw, fe_fb, fe_part, cv_col;
     int fe_mels = 0;
     DevBuf lg_part;  // per-workgroup (max, index) partials of the fused logits argmax
     // RoPE frequency table of the last (rope_base, head_dim) the _dev entry saw
@@ -1312,42 +1312,26 @@ int upload_table(vokra_hip_ctx* c, DevBuf& b, const std::vector<float>& h) {
 
 // log_mel of `batch` clips of n_samples each (device), out [batch][n_mels][3000].
 int run_log_mel(vokra_hip_ctx* c, const float* d_pcm, size_t batch, size_t n_samples, size_t n_mels, float* d_out) {
-    const int NFR = vk::fe_n_frames(), NB = vk::fe_n_bins(), NFFT = vk::fe_n_fft();
     if (!c->fe_win.p) {
-        std::vector<float> w, b;
+        std::vector<float> w, t;
         vk::fe_hann_periodic(w);
-        vk::fe_dft_basis(b);
+        vk::fe_twiddles(t);
         int st = upload_table(c, c->fe_win, w);
-        if (!st) st = upload_table(c, c->fe_basis, b);
+        if (!st) st = upload_table(c, c->fe_tw, t);
         if (st) return st;
     }
     if (c->fe_mels != (int)n_mels) {
-        std::vector<float> fb;
+        std::vector<float> fb, packed;
         vk::fe_mel_filterbank((int)n_mels, fb);
-        int st = upload_table(c, c->fe_fb, fb);
+        vk::fe_mel_ranges((int)n_mels, fb, packed);
+        int st = upload_table(c, c->fe_fb, packed);
         if (st) return st;
         c->fe_mels = (int)n_mels;
     }
-    const size_t rows = batch * (size_t)NFR;
-    VK_TRY(c->fe_frames.ensure(rows * NFFT * sizeof(float)), "hipMalloc(frames)");
-    VK_TRY(c->fe_spec.ensure(rows * 2 * NB * sizeof(float)), "hipMalloc(spectrum)");
-    VK_TRY(c->fe_pow.ensure(rows * NB * sizeof(float)), "hipMalloc(power)");
-    VK_TRY(c->fe_mel.ensure(rows * n_mels * sizeof(float)), "hipMalloc(mel)");
     VK_TRY(c->fe_part.ensure(batch * vk::logmel_n_partial() * sizeof(float)), "hipMalloc(partials)");
-    float* frames = (float*)c->fe_frames.p;
-    VK_TRY(vk::launch_stft_frames(c->stream, d_pcm, (int)batch, (int)n_samples, (const float*)c->fe_win.p, frames),
-           "launch(vk_stft_frames)");
-    VK_TRY(vk::launch_gemm_f32(c->stream, true, frames, (const float*)c->fe_basis.p, nullptr, (float*)c->fe_spec.p,
-                               (int)rows, 2 * NB, NFFT),
-           "launch(vk_gemm_f32 stft)");
-    VK_TRY(vk::launch_power_spec(c->stream, (const float*)c->fe_spec.p, (float*)c->fe_pow.p, rows),
-           "launch(vk_power_spec)");
-    VK_TRY(vk::launch_gemm_f32(c->stream, true, (const float*)c->fe_pow.p, (const float*)c->fe_fb.p, nullptr,
-                               (float*)c->fe_mel.p, (int)rows, (int)n_mels, NB),
-           "launch(vk_gemm_f32 mel)");
-    VK_TRY(vk::launch_logmel_finish(c->stream, (const float*)c->fe_mel.p, (int)batch, (int)n_mels, d_out,
-                                    (float*)c->fe_part.p),
-           "launch(vk_logmel)");
+    VK_TRY(vk::launch_log_mel(c->stream, d_pcm, (int)batch, (int)n_samples, (int)n_mels, (const float*)c->fe_win.p,
+                              (const float*)c->fe_tw.p, (const float*)c->fe_fb.p, d_out, (float*)c->fe_part.p),
+           "launch(vk_log_mel)");
     return VOKRA_HIP_OK;
 }
 
@@ -1784,8 +1768,8 @@ void vokra_hip_destroy(vokra_hip_ctx_t* c) {
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
     for (DevBuf* b : {&c->in0, &c->in1, &c->in2, &c->out0, &c->act.frag, &c->act.scale, &c->act.gsum, &c->at_qh,
-                      &c->at_ql, &c->at_kh, &c->at_kl, &c->at_vh, &c->at_vl, &c->at_po, &c->at_pml, &c->fe_win, &c->fe_basis, &c->fe_fb,
-                      &c->fe_frames, &c->fe_spec, &c->fe_pow, &c->fe_mel, &c->fe_part, &c->cv_col, &c->lg_part,
+                      &c->at_ql, &c->at_kh, &c->at_kl, &c->at_vh, &c->at_vl, &c->at_po, &c->at_pml, &c->fe_win, &c->fe_tw, &c->fe_fb,
+                      &c->fe_part, &c->cv_col, &c->lg_part,
                       &c->rope_theta, &c->rope_pos})
         b->release();
     (void)hipStreamDestroy(c->stream);
@@ -2395,8 +2379,8 @@ int vokra_hip_conv1d_f32_dev(vokra_hip_ctx_t* c, const float* d_in, size_t in_ch
     if (!d_out || !d_w || (in_ch && !d_in)) return fail(VOKRA_HIP_ERROR_INVALID_ARGUMENT, "conv1d: NULL buffer");
     VK_TRY(set_dev(c), "hipSetDevice");
     VK_TRY(c->cv_col.ensure(col_n * sizeof(float) + 16), "hipMalloc(im2col)");
-    VK_TRY(vk::launch_im2col(c->stream, false, d_in, 0, in_len, 1, 1, (int)in_ch, (int)in_len, (int)kernel, (int)stride,
-                             (int)padding, (int)out_len, (float*)c->cv_col.p),
+    VK_TRY(vk::launch_im2col(c->stream, d_in, (int)in_ch, (int)in_len, (int)kernel, (int)stride, (int)padding,
+                             (int)out_len, (float*)c->cv_col.p),
            "launch(vk_im2col)");
     VK_TRY(vk::launch_gemm_f32(c->stream, false, d_w, (const float*)c->cv_col.p, nullptr, d_out, (int)out_ch,
                                (int)out_len, (int)kk),

@@ -4,13 +4,14 @@
 // (crates/vokra-backend-cpu/src/kernels/mod.rs:583-822) for the encoder's conv
 // stem (crates/vokra-models/src/whisper/encoder.rs:58-108).
 //
-// The STFT is a GEMM: every 400-sample frame (reflect-padded, windowed) times a
-// [402 x 400] basis of cos / sin rows gives the 201 complex bins; the power
-// spectrum times the [n_mels x 201] filter bank is a second GEMM; both run on
-// the f32 matrix-core GEMM (vk_gemm_f32). log10, the per-clip maximum and the
-// (max(v, gmax - 8) + 4) / 4 normalisation follow in two small passes.
-// Convolution is im2col + the same GEMM.
+// The log-mel is one pass from samples to log10 energies (a real FFT per frame in
+// LDS, the power spectrum, the filter bank's nonzero weights) and one for the
+// per-clip (max(v, gmax - 8) + 4) / 4 normalisation. Convolution is im2col + the
+// f32 matrix-core GEMM (the encoder's conv stem has kernels of its own,
+// vk_stem.hip).
+#include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 #include "vk_common.h"
@@ -19,58 +20,160 @@ namespace vk {
 
 namespace fe {
 constexpr int NS = 480000, NFFT = 400, HOP = 160, NFR = 3000, NB = 201, PAD = 200;
-constexpr int LOG_ROWS = 16;  // frames per workgroup of the log pass
+constexpr int FR = 16;              // frames per workgroup of the transform
+constexpr int NC = NFFT / 2;        // complex points
+constexpr int PW = 205;             // floats per frame's power row (odd: frames on distinct banks)
 }  // namespace fe
 
 // numpy mode="reflect" (crates/vokra-ops/src/stft.rs:269-285) for the
 // single reflection the 200-sample centre padding needs.
 __device__ __forceinline__ int fe_reflect(int i, int n) { return i < 0 ? -i : (i >= n ? 2 * (n - 1) - i : i); }
 
-// frames[b * 3000 + t][i] = clip_b[reflect(160 t + i - 200)] * window[i], the
-// clip zero-padded / trimmed to 480000 samples (mel.rs:134-137, fused_logmel.rs:135-138).
-__global__ void vk_stft_frames(const float* __restrict__ pcm, int n_samples, const float* __restrict__ win,
-                               float* __restrict__ frames, int batch) {
-    const size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t total = (size_t)batch * fe::NFR * fe::NFFT;
-    if (gid >= total) return;
-    const int i = (int)(gid % fe::NFFT);
-    const size_t bt = gid / fe::NFFT;
-    const int t = (int)(bt % fe::NFR), b = (int)(bt / fe::NFR);
-    const int q = fe_reflect(t * fe::HOP + i - fe::PAD, fe::NS);
-    const float x = q < n_samples ? pcm[(size_t)b * n_samples + q] : 0.0f;
-    frames[gid] = x * win[i];
+__device__ __forceinline__ float2 fe_add(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
+__device__ __forceinline__ float2 fe_sub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
+__device__ __forceinline__ float2 fe_mul(float2 a, float2 b) {
+    return make_float2(fmaf(a.x, b.x, -(a.y * b.y)), fmaf(a.x, b.y, a.y * b.x));
+}
+__device__ __forceinline__ float2 fe_mul_mi(float2 a) { return make_float2(a.y, -a.x); }  // * -i
+
+// Forward DFT of 4 / 8 / 5 points in place (natural order in and out).
+__device__ __forceinline__ void fe_dft4(float2& a, float2& b, float2& c, float2& d) {
+    const float2 s0 = fe_add(a, c), s1 = fe_sub(a, c), s2 = fe_add(b, d), s3 = fe_mul_mi(fe_sub(b, d));
+    a = fe_add(s0, s2);
+    b = fe_add(s1, s3);
+    c = fe_sub(s0, s2);
+    d = fe_sub(s1, s3);
+}
+__device__ __forceinline__ void fe_dft8(float2 (&x)[8]) {
+    float2 e[4] = {x[0], x[2], x[4], x[6]}, o[4] = {x[1], x[3], x[5], x[7]};
+    fe_dft4(e[0], e[1], e[2], e[3]);
+    fe_dft4(o[0], o[1], o[2], o[3]);
+    const float h = 0.70710678118654752440f;
+    o[1] = make_float2(h * (o[1].x + o[1].y), h * (o[1].y - o[1].x));   // * exp(-i pi / 4)
+    o[2] = fe_mul_mi(o[2]);
+    o[3] = make_float2(h * (o[3].y - o[3].x), -h * (o[3].x + o[3].y));  // * exp(-3 i pi / 4)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        x[k] = fe_add(e[k], o[k]);
+        x[k + 4] = fe_sub(e[k], o[k]);
+    }
+}
+__device__ __forceinline__ void fe_dft5(float2 (&x)[5]) {
+    const float c1 = 0.30901699437494742410f, c2 = -0.80901699437494742410f;  // cos(2 pi / 5), cos(4 pi / 5)
+    const float s1 = 0.95105651629515357212f, s2 = 0.58778525229247312917f;   // sin
+    const float2 a = fe_add(x[1], x[4]), b = fe_add(x[2], x[3]), d = fe_sub(x[1], x[4]), f = fe_sub(x[2], x[3]);
+    const float2 u1 = make_float2(fmaf(c2, b.x, fmaf(c1, a.x, x[0].x)), fmaf(c2, b.y, fmaf(c1, a.y, x[0].y)));
+    const float2 u2 = make_float2(fmaf(c1, b.x, fmaf(c2, a.x, x[0].x)), fmaf(c1, b.y, fmaf(c2, a.y, x[0].y)));
+    const float2 v1 = make_float2(fmaf(s2, f.x, s1 * d.x), fmaf(s2, f.y, s1 * d.y));
+    const float2 v2 = make_float2(fmaf(-s1, f.x, s2 * d.x), fmaf(-s1, f.y, s2 * d.y));
+    x[0] = fe_add(x[0], fe_add(a, b));
+    x[1] = make_float2(u1.x + v1.y, u1.y - v1.x);
+    x[4] = make_float2(u1.x - v1.y, u1.y + v1.x);
+    x[2] = make_float2(u2.x + v2.y, u2.y - v2.x);
+    x[3] = make_float2(u2.x - v2.y, u2.y + v2.x);
 }
 
-// power[r][k] = re^2 + im^2 of the spectrum rows [re 0..200 | im 0..200].
-__global__ void vk_power_spec(const float* __restrict__ spec, float* __restrict__ power, size_t rows) {
-    const size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= rows * fe::NB) return;
-    const size_t r = gid / fe::NB;
-    const int k = (int)(gid % fe::NB);
-    const float re = spec[r * (2 * fe::NB) + k], im = spec[r * (2 * fe::NB) + fe::NB + k];
-    power[gid] = re * re + im * im;
-}
-
-// out[b][m][t] = log10(max(mel[b * 3000 + t][m], 1e-10)); one workgroup per
-// (clip, 16 frames) writes its partial maximum to partial[b][wg].
-__global__ __launch_bounds__(256) void vk_logmel_log(const float* __restrict__ mel, int n_mels,
-                                                     float* __restrict__ out, float* __restrict__ partial) {
+// out[b][m][t] = log10(max(mel energy, 1e-10)) of frame t of clip b (zero-padded
+// / trimmed to 480000 samples, reflect-padded by 200, windowed: mel.rs:134-137,
+// fused_logmel.rs:135-138), FR frames per workgroup, and the workgroup's maximum
+// into partial[b][wg].
+// Bound: LDS and arithmetic of a few thousand flops per frame; the samples and
+// the result are 1.9 + 1.5 MB per clip. A 400-point real transform is a 200-point
+// complex one of (even, odd) samples, 200 = 8 x 25 as eight 25-point sequences:
+// 8-point transforms over n = 25 n1 + n2, twiddles W200^(n2 k1), then 25 = 5 x 5,
+// every pass in place in LDS (25 k1 + 5 c + d holds bin k1 + 8 (c + 5 d) at the
+// end). It replaces a 402 x 400 f32 GEMM over materialised frames, a dense
+// filter-bank GEMM and the passes between them: log-mel of 4 clips, 128 bands,
+// 114 -> 25 us, and its rounding error is that of ~10 stages, not of 400-term sums:
+// relative 2-norm of the result against 64 bits 1.5e-7, the GEMMs 2.6e-7.
+// fb: per band {first bin, end bin} as ints, then the dense [n_mels][201] weights.
+__global__ __launch_bounds__(256) void vk_log_mel(const float* __restrict__ pcm, int n_samples,
+                                                  const float* __restrict__ win, const float2* __restrict__ tw_g,
+                                                  const float* __restrict__ fb, int n_mels, float* __restrict__ out,
+                                                  float* __restrict__ partial) {
+    using namespace fe;
+    __shared__ float2 z[FR][NC];
+    __shared__ float pw[FR][PW];
+    __shared__ float2 tw[NFFT];  // W400^j
     __shared__ float red[4];
-    const int b = blockIdx.y, t0 = blockIdx.x * fe::LOG_ROWS;
+    const int tid = threadIdx.x, b = blockIdx.y, t0 = blockIdx.x * FR;
+    const float* clip = pcm + (size_t)b * n_samples;
+    for (int i = tid; i < NFFT; i += 256) tw[i] = tw_g[i];
+    for (int i = tid; i < FR * NC; i += 256) {
+        const int f = i / NC, n = i - f * NC, t = t0 + f;
+        float2 v = make_float2(0.0f, 0.0f);
+        if (t < NFR) {
+            const int p0 = fe_reflect(t * HOP + 2 * n - PAD, NS), p1 = fe_reflect(t * HOP + 2 * n + 1 - PAD, NS);
+            v.x = (p0 < n_samples ? clip[p0] : 0.0f) * win[2 * n];
+            v.y = (p1 < n_samples ? clip[p1] : 0.0f) * win[2 * n + 1];
+        }
+        z[f][n] = v;
+    }
+    __syncthreads();
+    for (int i = tid; i < FR * 25; i += 256) {
+        const int f = i / 25, n2 = i - f * 25;
+        float2 x[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) x[q] = z[f][25 * q + n2];
+        fe_dft8(x);
+        z[f][n2] = x[0];
+#pragma unroll
+        for (int q = 1; q < 8; ++q) z[f][25 * q + n2] = fe_mul(x[q], tw[2 * n2 * q]);  // W200^(n2 q), 2 * 24 * 7 < 400
+    }
+    __syncthreads();
+    for (int i = tid; i < FR * 40; i += 256) {
+        const int f = i / 40, r = i - f * 40, k1 = r / 5, q = r - k1 * 5;
+        float2* s = &z[f][25 * k1 + q];
+        float2 x[5];
+#pragma unroll
+        for (int a = 0; a < 5; ++a) x[a] = s[5 * a];
+        fe_dft5(x);
+        s[0] = x[0];
+#pragma unroll
+        for (int c = 1; c < 5; ++c) s[5 * c] = fe_mul(x[c], tw[16 * q * c]);  // W25^(q c), 16 * 16 < 400
+    }
+    __syncthreads();
+    for (int i = tid; i < FR * 40; i += 256) {
+        const int f = i / 40, r = i - f * 40;
+        float2* s = &z[f][5 * r];
+        float2 x[5] = {s[0], s[1], s[2], s[3], s[4]};
+        fe_dft5(x);
+#pragma unroll
+        for (int a = 0; a < 5; ++a) s[a] = x[a];
+    }
+    __syncthreads();
+    // X[k] = (Z[k] + conj Z[200 - k]) / 2 - i W400^k (Z[k] - conj Z[200 - k]) / 2, and X[200 - k] from the same two
+    for (int i = tid; i < FR * 101; i += 256) {
+        const int f = i / 101, k = i - f * 101, kr = k == 0 ? 0 : NC - k;
+        auto at = [](int q) {
+            const int k1 = q & 7, k2 = q >> 3, d = k2 / 5;
+            return 25 * k1 + 5 * (k2 - 5 * d) + d;
+        };
+        const float2 u = z[f][at(k)], v = z[f][at(kr)];
+        const float2 e = make_float2(0.5f * (u.x + v.x), 0.5f * (u.y - v.y));
+        const float2 o = fe_mul(make_float2(0.5f * (u.y + v.y), 0.5f * (v.x - u.x)), tw[k]);
+        const float2 p = fe_add(e, o), m = fe_sub(e, o);
+        pw[f][k] = fmaf(p.x, p.x, p.y * p.y);
+        pw[f][NC - k] = fmaf(m.x, m.x, m.y * m.y);
+    }
+    __syncthreads();
+    const int2* range = reinterpret_cast<const int2*>(fb);
+    const float* w = fb + 2 * n_mels;
     float mx = -INFINITY;
-    for (int idx = threadIdx.x; idx < fe::LOG_ROWS * n_mels; idx += 256) {
-        const int m = idx / fe::LOG_ROWS, t = t0 + idx % fe::LOG_ROWS;  // consecutive threads: consecutive t
-        if (t >= fe::NFR) continue;
-        const float v = mel[((size_t)b * fe::NFR + t) * n_mels + m];
+    for (int i = tid; i < FR * n_mels; i += 256) {
+        const int f = i % FR, m = i / FR, t = t0 + f;  // consecutive threads: consecutive frames
+        if (t >= NFR) continue;
+        const int2 rg = range[m];
+        float v = 0.0f;
+        for (int k = rg.x; k < rg.y; ++k) v = fmaf(pw[f][k], w[(size_t)m * NB + k], v);
         const float l = log10f(v > 1e-10f ? v : 1e-10f);
-        out[((size_t)b * n_mels + m) * fe::NFR + t] = l;
+        out[((size_t)b * n_mels + m) * NFR + t] = l;
         mx = fmaxf(mx, l);
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, VK_WAVE));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
+    mx = vk_group_maxf<64>(mx);
+    if ((tid & 63) == 0) red[tid >> 6] = mx;
     __syncthreads();
-    if (threadIdx.x == 0) partial[(size_t)b * gridDim.x + blockIdx.x] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    if (tid == 0) partial[(size_t)b * gridDim.x + blockIdx.x] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
 }
 
 // out = (max(out, gmax - 8) + 4) / 4 with gmax the clip's maximum (every
@@ -88,34 +191,32 @@ __global__ __launch_bounds__(256) void vk_logmel_norm(float* __restrict__ out, i
     const float floor_v = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])) - 8.0f;
     const size_t n = (size_t)n_mels * fe::NFR;
     float* o = out + (size_t)b * n;
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256)
-        o[i] = (fmaxf(o[i], floor_v) + 4.0f) / 4.0f;
+    const size_t i0 = (size_t)blockIdx.x * 256 + threadIdx.x, step = (size_t)gridDim.x * 256;
+    if ((reinterpret_cast<uintptr_t>(out) & 15) == 0) {  // n is a multiple of 4
+        float4* o4 = reinterpret_cast<float4*>(o);
+        for (size_t i = i0; i < n / 4; i += step) {
+            float4 v = o4[i];
+            v.x = (fmaxf(v.x, floor_v) + 4.0f) / 4.0f;
+            v.y = (fmaxf(v.y, floor_v) + 4.0f) / 4.0f;
+            v.z = (fmaxf(v.z, floor_v) + 4.0f) / 4.0f;
+            v.w = (fmaxf(v.w, floor_v) + 4.0f) / 4.0f;
+            o4[i] = v;
+        }
+        return;
+    }
+    for (size_t i = i0; i < n; i += step) o[i] = (fmaxf(o[i], floor_v) + 4.0f) / 4.0f;
 }
 
-// im2col over x(b, c, p) = x[b * sb + c * sc + p * sp] (zero outside 0..in_len):
-// TRANS: col[b * out_len + t][c * kernel + kk]; else col[c * kernel + kk][t]
-// (batch 1), the reference's layout (mod.rs:794-806).
-template <bool TRANS>
-__global__ void vk_im2col(const float* __restrict__ x, size_t sb, size_t sc, size_t sp, int batch, int in_ch,
-                          int in_len, int kernel, int stride, int padding, int out_len, float* __restrict__ col) {
+// im2col of x [in_ch][in_len] (zero outside 0..in_len): col[c * kernel + kk][t],
+// the reference's layout (mod.rs:794-806).
+__global__ void vk_im2col(const float* __restrict__ x, int in_ch, int in_len, int kernel, int stride, int padding,
+                          int out_len, float* __restrict__ col) {
     const size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t kk_total = (size_t)in_ch * kernel;
-    const size_t total = (size_t)batch * out_len * kk_total;
-    if (gid >= total) return;
-    size_t row, t, b, r;
-    if (TRANS) {
-        r = gid % kk_total;
-        row = gid / kk_total;  // b * out_len + t
-        t = row % out_len;
-        b = row / out_len;
-    } else {
-        t = gid % out_len;
-        r = gid / out_len;
-        b = 0;
-    }
-    const int c = (int)(r / kernel), kk = (int)(r % kernel);
-    const long pos = (long)t * stride + kk - padding;
-    col[gid] = (pos >= 0 && pos < in_len) ? x[b * sb + c * sc + (size_t)pos * sp] : 0.0f;
+    if (gid >= (size_t)out_len * in_ch * kernel) return;
+    const size_t t = gid % out_len, r = gid / out_len;
+    const size_t c = r / kernel;
+    const long pos = (long)t * stride + (long)(r % kernel) - padding;
+    col[gid] = (pos >= 0 && pos < in_len) ? x[c * in_len + (size_t)pos] : 0.0f;
 }
 
 // out[oc][t] += bias[oc] (the reference adds the bias after its GEMM, mod.rs:814-820).
@@ -124,21 +225,6 @@ __global__ void vk_add_row_bias(float* __restrict__ out, const float* __restrict
     if (gid >= (size_t)rows * cols) return;
     out[gid] = out[gid] + bias[gid / cols];
 }
-
-// out[r][c] = out[r][c] + pos[r % period][c] (encoder.rs:98-104: conv output
-// plus positional embedding, per clip of a batch).
-__global__ void vk_add_pos(float* __restrict__ out, const float* __restrict__ pos, size_t rows, int d, int period) {
-    const size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= rows * d) return;
-    const size_t r = gid / d;
-    const int c = (int)(gid % d);
-    out[gid] = out[gid] + pos[(r % period) * d + c];
-}
-
-template __global__ void vk_im2col<true>(const float*, size_t, size_t, size_t, int, int, int, int, int, int, int,
-                                         float*);
-template __global__ void vk_im2col<false>(const float*, size_t, size_t, size_t, int, int, int, int, int, int, int,
-                                          float*);
 
 // ---------------------------------------------------------------------------
 // Host-side tables (built once per context, in double, cast to f32 as the
@@ -153,15 +239,14 @@ void fe_hann_periodic(std::vector<float>& w) {
     }
 }
 
-// DFT basis rows: k-th cos row, then k-th -sin row (k = 0..200).
-void fe_dft_basis(std::vector<float>& b) {
-    b.assign((size_t)2 * fe::NB * fe::NFFT, 0.0f);
-    for (int k = 0; k < fe::NB; ++k)
-        for (int n = 0; n < fe::NFFT; ++n) {
-            const double th = 2.0 * M_PI * (double)((k * n) % fe::NFFT) / (double)fe::NFFT;
-            b[(size_t)k * fe::NFFT + n] = (float)std::cos(th);
-            b[(size_t)(fe::NB + k) * fe::NFFT + n] = (float)-std::sin(th);
-        }
+// W400^j = exp(-2 pi i j / 400), j = 0 .. 399, as (cos, -sin) pairs.
+void fe_twiddles(std::vector<float>& t) {
+    t.resize(2 * fe::NFFT);
+    for (int j = 0; j < fe::NFFT; ++j) {
+        const double th = 2.0 * M_PI * (double)j / (double)fe::NFFT;
+        t[2 * j] = (float)std::cos(th);
+        t[2 * j + 1] = (float)-std::sin(th);
+    }
 }
 
 // Slaney mel scale and the filter bank of crates/vokra-ops/src/mel.rs:29-130
@@ -194,44 +279,43 @@ void fe_mel_filterbank(int n_mels, std::vector<float>& w) {
     }
 }
 
+// The filter bank as vk_log_mel reads it: per band its first and end nonzero
+// bin (the bits of two ints; an empty band 0, 0), then the dense weights.
+void fe_mel_ranges(int n_mels, const std::vector<float>& w, std::vector<float>& packed) {
+    packed.assign(2 * (size_t)n_mels, 0.0f);
+    for (int m = 0; m < n_mels; ++m) {
+        int lo = fe::NB, hi = 0;
+        for (int k = 0; k < fe::NB; ++k)
+            if (w[(size_t)m * fe::NB + k] != 0.0f) {
+                lo = std::min(lo, k);
+                hi = k + 1;
+            }
+        if (hi == 0) lo = 0;
+        std::memcpy(&packed[2 * m], &lo, 4);
+        std::memcpy(&packed[2 * m + 1], &hi, 4);
+    }
+    packed.insert(packed.end(), w.begin(), w.end());
+}
+
 int fe_n_frames() { return fe::NFR; }
-int fe_n_bins() { return fe::NB; }
-int fe_n_fft() { return fe::NFFT; }
 
-hipError_t launch_stft_frames(hipStream_t s, const float* pcm, int batch, int n_samples, const float* win,
-                              float* frames) {
-    const size_t total = (size_t)batch * fe::NFR * fe::NFFT;
-    hipLaunchKernelGGL(vk_stft_frames, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, pcm, n_samples, win,
-                       frames, batch);
-    return hipGetLastError();
-}
+int logmel_n_partial() { return (fe::NFR + fe::FR - 1) / fe::FR; }
 
-hipError_t launch_power_spec(hipStream_t s, const float* spec, float* power, size_t rows) {
-    hipLaunchKernelGGL(vk_power_spec, dim3((unsigned)((rows * fe::NB + 255) / 256)), dim3(256), 0, s, spec, power,
-                       rows);
-    return hipGetLastError();
-}
-
-int logmel_n_partial() { return (fe::NFR + fe::LOG_ROWS - 1) / fe::LOG_ROWS; }
-
-hipError_t launch_logmel_finish(hipStream_t s, const float* mel, int batch, int n_mels, float* out, float* partial) {
+hipError_t launch_log_mel(hipStream_t s, const float* pcm, int batch, int n_samples, int n_mels, const float* win,
+                          const float* tw, const float* fb, float* out, float* partial) {
     const int np = logmel_n_partial();
-    hipLaunchKernelGGL(vk_logmel_log, dim3(np, batch), dim3(256), 0, s, mel, n_mels, out, partial);
-    hipLaunchKernelGGL(vk_logmel_norm, dim3(64, batch), dim3(256), 0, s, out, n_mels, partial, np);
+    hipLaunchKernelGGL(vk_log_mel, dim3(np, batch), dim3(256), 0, s, pcm, n_samples, win,
+                       reinterpret_cast<const float2*>(tw), fb, n_mels, out, partial);
+    hipLaunchKernelGGL(vk_logmel_norm, dim3(128, batch), dim3(256), 0, s, out, n_mels, partial, np);
     return hipGetLastError();
 }
 
-hipError_t launch_im2col(hipStream_t s, bool trans, const float* x, size_t sb, size_t sc, size_t sp, int batch,
-                         int in_ch, int in_len, int kernel, int stride, int padding, int out_len, float* col) {
-    const size_t total = (size_t)batch * out_len * in_ch * kernel;
+hipError_t launch_im2col(hipStream_t s, const float* x, int in_ch, int in_len, int kernel, int stride, int padding,
+                         int out_len, float* col) {
+    const size_t total = (size_t)out_len * in_ch * kernel;
     if (total == 0) return hipSuccess;
-    const dim3 grid((unsigned)((total + 255) / 256));
-    if (trans)
-        hipLaunchKernelGGL(vk_im2col<true>, grid, dim3(256), 0, s, x, sb, sc, sp, batch, in_ch, in_len, kernel, stride,
-                           padding, out_len, col);
-    else
-        hipLaunchKernelGGL(vk_im2col<false>, grid, dim3(256), 0, s, x, sb, sc, sp, batch, in_ch, in_len, kernel, stride,
-                           padding, out_len, col);
+    hipLaunchKernelGGL(vk_im2col, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, x, in_ch, in_len, kernel,
+                       stride, padding, out_len, col);
     return hipGetLastError();
 }
 
@@ -239,13 +323,6 @@ hipError_t launch_add_row_bias(hipStream_t s, float* out, const float* bias, int
     const size_t total = (size_t)rows * cols;
     if (total == 0) return hipSuccess;
     hipLaunchKernelGGL(vk_add_row_bias, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, out, bias, rows, cols);
-    return hipGetLastError();
-}
-
-hipError_t launch_add_pos(hipStream_t s, float* out, const float* pos, size_t rows, int d, int period) {
-    const size_t total = rows * d;
-    if (total == 0) return hipSuccess;
-    hipLaunchKernelGGL(vk_add_pos, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, out, pos, rows, d, period);
     return hipGetLastError();
 }
 

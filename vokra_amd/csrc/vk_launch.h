@@ -408,23 +408,21 @@ void qact_outputs_written(vokra_hip_qact* qa, size_t m, int act_quant);
 }  // namespace vk
 
 namespace vk {
-// Whisper front end (vk_frontend.hip): frame grid 3000 x 400, 201 bins.
+// Whisper front end (vk_frontend.hip): 3000 frames of 400 samples, 201 bins.
 int fe_n_frames();
-int fe_n_bins();
-int fe_n_fft();
 int logmel_n_partial();
 }  // namespace vk
 #include <vector>
 namespace vk {
 void fe_hann_periodic(std::vector<float>& w);
-void fe_dft_basis(std::vector<float>& b);
+void fe_twiddles(std::vector<float>& t);
 void fe_mel_filterbank(int n_mels, std::vector<float>& w);
-hipError_t launch_stft_frames(hipStream_t s, const float* pcm, int batch, int n_samples, const float* win,
-                              float* frames);
-hipError_t launch_power_spec(hipStream_t s, const float* spec, float* power, size_t rows);
-hipError_t launch_logmel_finish(hipStream_t s, const float* mel, int batch, int n_mels, float* out, float* partial);
-hipError_t launch_im2col(hipStream_t s, bool trans, const float* x, size_t sb, size_t sc, size_t sp, int batch,
-                         int in_ch, int in_len, int kernel, int stride, int padding, int out_len, float* col);
+// Samples -> normalised log-mel [batch][n_mels][3000]; tw: fe_twiddles, fb: fe_mel_filterbank with its bands' bin
+// ranges (fe_mel_ranges), partial: batch * logmel_n_partial() floats.
+void fe_mel_ranges(int n_mels, const std::vector<float>& w, std::vector<float>& packed);
+hipError_t launch_log_mel(hipStream_t s, const float* pcm, int batch, int n_samples, int n_mels, const float* win,
+                          const float* tw, const float* fb, float* out, float* partial);
+hipError_t launch_im2col(hipStream_t s, const float* x, int in_ch, int in_len, int kernel, int stride, int padding,
+                         int out_len, float* col);
 hipError_t launch_add_row_bias(hipStream_t s, float* out, const float* bias, int rows, int cols);
-hipError_t launch_add_pos(hipStream_t s, float* out, const float* pos, size_t rows, int d, int period);
 }  // namespace vk
