@@ -128,6 +128,11 @@ __device__ __forceinline__ int vk_row_bcast_i(int v) {
     return __builtin_amdgcn_mov_dpp(v, 0x150 + J, 0xf, 0xf, true);
 }
 
+// component s (a constant after unrolling) of a float4
+__device__ __forceinline__ float vk_f4c(const float4& v, int s) {
+    return s == 0 ? v.x : (s == 1 ? v.y : (s == 2 ? v.z : v.w));
+}
+
 // Max-reduce over groups of `G` consecutive lanes (G power of two <= 64);
 // every lane of a group ends with the group's value. The inputs must be
 // +0 or positive and not NaN (the callers reduce fmaxf(0, |x|), which maps a

@@ -96,10 +96,6 @@ __global__ __launch_bounds__(256) void vk_gemm_f32(const float* __restrict__ a, 
             }
 }
 
-__device__ __forceinline__ float vk_f4c(const float4& v, int s) {
-    return s == 0 ? v.x : (s == 1 ? v.y : (s == 2 ? v.z : v.w));
-}
-
 // Tiled GEMM for K % 16 == 0: 128 x 128 workgroup tiles (four 64 x 64 waves),
 // K in 16-wide stages moved global -> LDS by direct loads through a ring of
 // three stages (two ahead of the MFMAs), XCD-aware tile order. Fragments of

@@ -1035,10 +1035,13 @@ __global__ __launch_bounds__(256, 5) void vk_paged_attn_w64(KvDev c, int layer, 
 //     K quants are exact fp16 integers, so each block dot is the exact integer
 //     dot against the two fp16 halves of q * scale; the key's f16 block scale
 //     is applied to the block sum (v_mfma_f32_16x16x32_f16, keys on the 16-row
-//     side, heads on the 16-column side, padded to 16);
+//     side, heads on the 16-column side);
 //   O^T[dim][head] += V^T . (p * d_v)^T
 //     the V block scale of each key folds into P, split hi/lo; V^T comes from
 //     a per-wave LDS copy of the tile converted to fp16.
+// With at most 8 heads the halves share one product: column h holds head h's hi
+// half and column h + 8 its lo half, and the two columns are added where a result
+// is needed (S per tile, O once), so both columns of a head carry the same softmax.
 //
 // Each wave owns the 32-key tiles j0 = k0 + 32 w + 128 i of the split and keeps
 // its own online softmax; the four states merge in wave order at the end.
@@ -1054,25 +1057,40 @@ static_assert((VROW * 2) % 16 == 0, "16-byte LDS reads of V^T rows");
 typedef _Float16 vk_h16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 vk_h16x2_t __attribute__((ext_vector_type(2)));
 
-// Two signed bytes (selected by `sel` from {hi_src:lo_src}) -> two exact fp16:
-// 0x64uu with u = x + 128 is the fp16 1024 + u; subtracting 1152 leaves x.
-__device__ __forceinline__ uint32_t vk_i8pair_f16(uint32_t hi_src, uint32_t lo_src, uint32_t sel) {
-    const uint32_t t = __builtin_amdgcn_perm(hi_src, lo_src, sel) ^ 0x64806480u;
-    vk_h16x2_t h = __builtin_bit_cast(vk_h16x2_t, t);
+// Four signed bytes biased to unsigned (x ^ 0x80808080) -> fp16. From one word: the
+// byte under 0x64 is the fp16 1024 + u, and 1152 less leaves x. From the same byte
+// of two words: the byte under 0x00 is the (subnormal) fp16 u * 2^-24; times 2^14,
+// less 128 * 2^-10, leaves x * 2^-10 (kVUnscale at the end takes it back). Both exact;
+// two instructions per pair, where shifting the bias in per pair takes three.
+constexpr float kVUnscale = 1024.0f;
+__device__ __forceinline__ uint32_t vk_u8pair_f16(uint32_t w, uint32_t sel) {
+    vk_h16x2_t h = __builtin_bit_cast(vk_h16x2_t, __builtin_amdgcn_perm(0x64646464u, w, sel));
     h = h + (vk_h16x2_t){(_Float16)-1152.0f, (_Float16)-1152.0f};
     return __builtin_bit_cast(uint32_t, h);
 }
+__device__ __forceinline__ uint32_t vk_u8cross_f16(uint32_t hi_src, uint32_t lo_src, uint32_t sel) {
+    const vk_h16x2_t h = __builtin_bit_cast(vk_h16x2_t, __builtin_amdgcn_perm(hi_src, lo_src, sel));
+    const vk_h16x2_t up = {(_Float16)16384.0f, (_Float16)16384.0f}, bias = {(_Float16)-0.125f, (_Float16)-0.125f};
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(h, up, bias));
+}
 // eight signed bytes (little-endian in w) -> eight fp16 in order
 __device__ __forceinline__ vk_h16x8_t vk_i8x8_f16(uint2 w) {
+    w.x ^= 0x80808080u;
+    w.y ^= 0x80808080u;
     uint4 r;
-    r.x = vk_i8pair_f16(0, w.x, 0x0c010c00u);
-    r.y = vk_i8pair_f16(0, w.x, 0x0c030c02u);
-    r.z = vk_i8pair_f16(0, w.y, 0x0c010c00u);
-    r.w = vk_i8pair_f16(0, w.y, 0x0c030c02u);
+    r.x = vk_u8pair_f16(w.x, 0x04010400u);
+    r.y = vk_u8pair_f16(w.x, 0x04030402u);
+    r.z = vk_u8pair_f16(w.y, 0x04010400u);
+    r.w = vk_u8pair_f16(w.y, 0x04030402u);
     return __builtin_bit_cast(vk_h16x8_t, r);
 }
 
-// two workgroups per CU (measured best: 29.3 vs 30.5 us at config 4)
+// Bound: latency and the load path together. 32 items of 512 .. 4096 keys, 16 heads
+// over 2 (us per layer with the combine, 25.6 before): 24.2; 8 us of it are the cache's
+// bytes, 6 the products and conversions, 13 launches and the chain lens -> pages ->
+// rows, which q's loads and conversion no longer extend (they ran before the first
+// page lookup: 1.1 us). 48 items, 64 heads over 8: 104 -> 91. Two workgroups per CU
+// (measured best: 29.3 vs 30.5 us at config 4); splits of 256 keys: 38 us.
 template <int G>
 __global__ __launch_bounds__(256, 2) void vk_paged_attn_gqa(KvDev c, int layer, const int* __restrict__ streams,
                                                          const int* __restrict__ lens, const float* __restrict__ q,
@@ -1083,7 +1101,7 @@ __global__ __launch_bounds__(256, 2) void vk_paged_attn_gqa(KvDev c, int layer, 
                                                          const float* __restrict__ ak, const float* __restrict__ av,
                                                          const int* __restrict__ at) {
     using namespace pg;
-    static_assert(G >= 2 && G <= 16, "query heads per kv head");
+    static_assert(G >= 2 && G <= 8, "query heads per kv head: their two halves fill the 16 columns");
     __shared__ __align__(16) _Float16 lvt[WAVES][HD][VROW];  // per wave: V^T of its tile (reused by the merge)
     __shared__ float lm[WAVES][16], ll[WAVES][16];
     static_assert(sizeof(lvt) >= sizeof(vk_f32x4) * (WAVES - 1) * (HD / 16) * 64, "merge buffer fits");
@@ -1134,48 +1152,65 @@ __global__ __launch_bounds__(256, 2) void vk_paged_attn_gqa(KvDev c, int layer, 
         }
     }
 
-    // q * scale of head hh (zero for padding heads) as the S^T B operand:
-    // lane (g, hh) holds dims 32b + 8g .. +7, split into fp16 hi + lo. With
-    // rope_cs, q is first rotated: dims j and j + 64 (blocks b and b + 2) sit
-    // in the same lane.
-    vk_h16x8_t qh[NB], ql[NB];
-    float x[NB][8];
+    // q * scale of the column's head (zero for padding heads) as the S^T B operand:
+    // lane (g, hh) holds dims 32b + 8g .. +7 of head hh % 8, the fp16 hi half in
+    // columns 0..7 and the lo half in columns 8..15. With rope_cs, q is first
+    // rotated: dims j and j + 64 (blocks b and b + 2) sit in the same lane.
+    vk_h16x8_t qh[NB];
+    const float lo_mask = hh >= 8 ? -1.0f : 0.0f;  // part = x + mask * hi: x itself, or what hi leaves of it
+    const int qhead = min(hh & 7, G - 1);  // padding heads load the last one, unused
+    float4 xq[NB][2], cs4[2][4];
+    auto load_q = [&]() {
+        const float4* qp = reinterpret_cast<const float4*>(q + ((size_t)item * hq + hk * G + qhead) * HD + 8 * g);
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) x[b][i] = 0.0f;
-        if (hh < G) {
-            const float4* qp =
-                reinterpret_cast<const float4*>(q + ((size_t)item * hq + hk * G + hh) * HD + 32 * b + 8 * g);
-            const float4 u = qp[0], v = qp[1];
-            x[b][0] = u.x; x[b][1] = u.y; x[b][2] = u.z; x[b][3] = u.w;
-            x[b][4] = v.x; x[b][5] = v.y; x[b][6] = v.z; x[b][7] = v.w;
+        for (int b = 0; b < NB; ++b) {
+            xq[b][0] = qp[8 * b];
+            xq[b][1] = qp[8 * b + 1];
         }
-    }
-    if (rope_cs && hh < G) {
-        static_assert(NB == 4, "the rotation pairs blocks b and b + 2");
+        if (rope_cs) {
+            static_assert(NB == 4, "the rotation pairs blocks b and b + 2");
+            const float4* cp = reinterpret_cast<const float4*>(rope_cs + (size_t)item * (HD / 2) + 8 * g);
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) cs4[b][i] = cp[16 * b + i];
+        }
+    };
+    auto prepare_q = [&]() {
+        float x[NB][8];
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) x[b][i] = vk_f4c(xq[b][i >> 2], i & 3);
+        if (rope_cs) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const float2 cs = make_float2(vk_f4c(cs4[b][i >> 1], 2 * (i & 1)), vk_f4c(cs4[b][i >> 1], 2 * (i & 1) + 1));
+                    const float a = x[b][i], bb = x[b + 2][i];
+                    x[b][i] = vk_rope_lo(a, bb, cs);
+                    x[b + 2][i] = vk_rope_hi(a, bb, cs);
+                }
+        }
+        bool bad = false;
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const float2 cs = rope_cs[(size_t)item * (HD / 2) + 32 * b + 8 * g + i];
-                const float a = x[b][i], bb = x[b + 2][i];
-                x[b][i] = vk_rope_lo(a, bb, cs);
-                x[b + 2][i] = vk_rope_hi(a, bb, cs);
+                float xs = (hh & 7) < G ? x[b][i] * scale : 0.0f;
+                asm("" : "+v"(xs));  // see the P operand below
+                bad |= vk_f16_overflow(xs);
+                const _Float16 h = (_Float16)xs;
+                float part = fmaf((float)h, lo_mask, xs);
+                asm("" : "+v"(part));
+                qh[b][i] = (_Float16)part;
             }
-    }
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const float xs = x[b][i] * scale;
-            if (vk_f16_overflow(xs)) atomicOr(&vk_kv_range_flag, 1u);
-            const _Float16 h = (_Float16)xs;
-            qh[b][i] = h;
-            ql[b][i] = (_Float16)(xs - (float)h);
-        }
-    }
+        if (bad) atomicOr(&vk_kv_range_flag, 1u);
+    };
     float m_run = -INFINITY, l_run = 0.0f;
+    float zero = 0.0f;
+    asm("" : "+v"(zero));  // not a constant: an fp16 operand converts for free in an FMA, not in a product
     vk_f32x4 o[HD / 16];
 #pragma unroll
     for (int et = 0; et < HD / 16; ++et) o[et] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -1188,27 +1223,42 @@ __global__ __launch_bounds__(256, 2) void vk_paged_attn_gqa(KvDev c, int layer, 
     // The loads of a tile: its page-table entries one tile ahead, its K / V
     // rows and block scales one tile ahead of the tile being computed.
     // Lane l looks up key l % 32 (lanes 32..63 repeat lanes 0..31). Every
-    // load is issued unconditionally (tile indices clamped to the wave's last
-    // tile, keys to the split's last key), so the wait before a tile's
-    // products counts only the younger loads and the prefetch stays in flight.
+    // load is issued unconditionally (pages clamped to the split's last, keys past
+    // the split read row 0), so the wait before a tile's products counts only the
+    // younger loads and the prefetch stays in flight.
     struct Tile {
         uint2 kw[2][NB];  // K operand rows: subtile n, row hh <-> key 8 (hh / 4) + 4 n + hh % 4
         uint4 vw[4];      // V rows of keys 4va + t, dims 16vc .. +15
         uint2 kd, vd;     // f16 block scales of key 8 (lane / 16) + lane % 8
         int has;          // that key is cached
     };
-    // the raw table entry of key lane % 32 of tile t (the key clamped into
-    // the split); load_tile masks keys past the split, so nothing here waits
-    auto page_of = [&](int t) -> int {
-        const int jk = jfirst + KT * WAVES * t + (lane & 31);
-        return c.table[trow + min(jk, k1 - 1) / c.bs];
+    // Key lane % 32 of a tile: its page index and place in the page, stepped from
+    // tile to tile (no division per tile).
+    struct Pos {
+        int page, in;
     };
-    auto load_tile = [&](int t, int raw) -> Tile {
+    const int step_page = KT * WAVES / c.bs, step_in = KT * WAVES % c.bs, last_page = max(k1 - 1, 0) / c.bs;
+    Pos pos;
+    pos.page = (jfirst + (lane & 31)) / c.bs;
+    pos.in = (jfirst + (lane & 31)) - pos.page * c.bs;
+    auto next_pos = [&](Pos x) -> Pos {
+        x.page += step_page;
+        x.in += step_in;
+        if (x.in >= c.bs) {
+            x.in -= c.bs;
+            ++x.page;
+        }
+        return x;
+    };
+    // its raw table entry (the page clamped into the split); load_tile masks
+    // keys past the split, so nothing here waits
+    auto page_of = [&](const Pos& x) -> int { return c.table[trow + min(x.page, last_page)]; };
+    const int slot0 = (s * c.nh + hk) * c.bs, page_slots = c.n_stream * c.nh * c.bs;  // head rows: 32 bits (the host checks)
+    auto load_tile = [&](int t, int raw, const Pos& x) -> Tile {
         Tile T;
         const int jk = jfirst + KT * WAVES * t + (lane & 31);
         const int pid = jk < k1 ? raw : -1;
-        const int slot_any = (int)kv_hrow(c, max(pid, 0), jk, s, hk);
-        const int slot = pid >= 0 ? slot_any : 0;  // row 0: in bounds, masked
+        const int slot = pid >= 0 ? pid * page_slots + slot0 + x.in : 0;  // row 0: in bounds, masked
 #pragma unroll
         for (int n = 0; n < 2; ++n) {
             const int sl = __shfl(slot, 8 * (hh >> 2) + 4 * n + (hh & 3), VK_WAVE);
@@ -1231,14 +1281,16 @@ __global__ __launch_bounds__(256, 2) void vk_paged_attn_gqa(KvDev c, int layer, 
         }
         return T;
     };
-    auto compute = [&](const Tile& T) {
-        // scales and presence of keys 8g + j (j = 4n + r) from the lanes that loaded them
+    // the value of the other column of this head (hi <-> lo): DPP row_ror 8
+    auto other_half = [](float v) {
+        return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x128, 0xf, 0xf, true));
+    };
+    auto compute = [&](const Tile& T, bool first) {
+        // scales of keys 8g + j (j = 4n + r) from the lanes that loaded them
         uint2 kds[8], vds[8];
-        int kval[8];
 #define VK_GQA_BC(J)                                                                                            \
         kds[J] = make_uint2((uint32_t)vk_row_bcast_i<J>((int)T.kd.x), (uint32_t)vk_row_bcast_i<J>((int)T.kd.y));   \
-        vds[J] = make_uint2((uint32_t)vk_row_bcast_i<J>((int)T.vd.x), (uint32_t)vk_row_bcast_i<J>((int)T.vd.y));   \
-        kval[J] = vk_row_bcast_i<J>(T.has);
+        vds[J] = make_uint2((uint32_t)vk_row_bcast_i<J>((int)T.vd.x), (uint32_t)vk_row_bcast_i<J>((int)T.vd.y));
         VK_GQA_BC(0) VK_GQA_BC(1) VK_GQA_BC(2) VK_GQA_BC(3) VK_GQA_BC(4) VK_GQA_BC(5) VK_GQA_BC(6) VK_GQA_BC(7)
 #undef VK_GQA_BC
 
@@ -1252,16 +1304,19 @@ __global__ __launch_bounds__(256, 2) void vk_paged_attn_gqa(KvDev c, int layer, 
                 const vk_h16x8_t a = vk_i8x8_f16(T.kw[n][b]);
                 vk_f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
                 d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qh[b], d, 0, 0, 0);
-                d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, ql[b], d, 0, 0, 0);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const uint2 kd = kds[4 * n + r];
-                    const uint32_t bits = (b < 2 ? kd.x : kd.y) >> (16 * (b & 1));
-                    acc[r] = fmaf(vk_f16_to_f32_hw(bits & 0xffffu), d[r], acc[r]);
+                    const vk_h16x2_t kd = __builtin_bit_cast(vk_h16x2_t, b < 2 ? kds[4 * n + r].x : kds[4 * n + r].y);
+                    acc[r] = fmaf((float)kd[b & 1], d[r], acc[r]);
                 }
             }
 #pragma unroll
-            for (int r = 0; r < 4; ++r) sc[4 * n + r] = kval[4 * n + r] ? acc[r] : -INFINITY;
+            for (int r = 0; r < 4; ++r) sc[4 * n + r] = acc[r] + other_half(acc[r]);
+        }
+        if (!__all(T.has)) {  // keys past the split or without a page
+#define VK_GQA_HAS(J) sc[J] = vk_row_bcast_i<J>(T.has) ? sc[J] : -INFINITY;
+            VK_GQA_HAS(0) VK_GQA_HAS(1) VK_GQA_HAS(2) VK_GQA_HAS(3) VK_GQA_HAS(4) VK_GQA_HAS(5) VK_GQA_HAS(6) VK_GQA_HAS(7)
+#undef VK_GQA_HAS
         }
 
         // ---- online softmax of head hh over the tile's 32 keys
@@ -1283,93 +1338,115 @@ __global__ __launch_bounds__(256, 2) void vk_paged_attn_gqa(KvDev c, int layer, 
         psum += __shfl_xor(psum, 32, VK_WAVE);
         l_run = l_run * alpha + psum;
         m_run = m_new;
+        if (!first) {  // (the first tile's O is zero)
 #pragma unroll
-        for (int et = 0; et < HD / 16; ++et)
+            for (int et = 0; et < HD / 16; ++et)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) o[et][r] *= alpha;
+                for (int r = 0; r < 4; ++r) o[et][r] *= alpha;
+        }
 
         // ---- V^T of the tile into this wave's LDS, as fp16 (keys 4va .. +3 of dim 16vc + x)
+        uint4 vw[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            vw[r] = make_uint4(T.vw[r].x ^ 0x80808080u, T.vw[r].y ^ 0x80808080u, T.vw[r].z ^ 0x80808080u, T.vw[r].w ^ 0x80808080u);
 #pragma unroll
         for (int x = 0; x < 16; ++x) {
             const int cw = x >> 2, sb = x & 3;  // component and byte of dim x in each row's 16 bytes
-            const uint4* vw = T.vw;
             const uint32_t w0 = cw == 0 ? vw[0].x : cw == 1 ? vw[0].y : cw == 2 ? vw[0].z : vw[0].w;
             const uint32_t w1 = cw == 0 ? vw[1].x : cw == 1 ? vw[1].y : cw == 2 ? vw[1].z : vw[1].w;
             const uint32_t w2 = cw == 0 ? vw[2].x : cw == 1 ? vw[2].y : cw == 2 ? vw[2].z : vw[2].w;
             const uint32_t w3 = cw == 0 ? vw[3].x : cw == 1 ? vw[3].y : cw == 2 ? vw[3].z : vw[3].w;
             const uint32_t sel = 0x0c000c00u | ((uint32_t)(4 + sb) << 16) | (uint32_t)sb;
             uint2 h;
-            h.x = vk_i8pair_f16(w1, w0, sel);
-            h.y = vk_i8pair_f16(w3, w2, sel);
+            h.x = vk_u8cross_f16(w1, w0, sel);
+            h.y = vk_u8cross_f16(w3, w2, sel);
             *reinterpret_cast<uint2*>(&lvt[wave][16 * vc + x][4 * va]) = h;
         }
 
         // ---- O^T += V^T . (p d_v)^T, one V block scale per pair of 16-dim tiles
 #pragma unroll
         for (int vb = 0; vb < NB; ++vb) {
-            vk_h16x8_t bh, bl;
+            vk_h16x8_t bp;  // hi, or lo = pd - hi: the mask keeps it branchless
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                const uint32_t bits = (vb < 2 ? vds[j].x : vds[j].y) >> (16 * (vb & 1));
-                const float pd = p[j] * vk_f16_to_f32_hw(bits & 0xffffu);
-                const _Float16 h = (_Float16)pd;
-                bh[j] = h;
-                bl[j] = (_Float16)(pd - (float)h);
+                const vk_h16x2_t d2 = __builtin_bit_cast(vk_h16x2_t, vb < 2 ? vds[j].x : vds[j].y);
+                float pd = fmaf(p[j], (float)d2[vb & 1], zero);  // the product, with the scale taken as fp16
+                // both columns must split the same f32 value: a conversion fused into
+                // the operation before it rounds once where the other column rounds
+                // twice, and hi + lo is then off by an fp16 ulp of hi
+                asm("" : "+v"(pd));
+                float part = fmaf((float)(_Float16)pd, lo_mask, pd);
+                asm("" : "+v"(part));
+                bp[j] = (_Float16)part;
             }
 #pragma unroll
             for (int e2 = 0; e2 < 2; ++e2) {
                 const int et = 2 * vb + e2;
                 const vk_h16x8_t a = *reinterpret_cast<const vk_h16x8_t*>(&lvt[wave][16 * et + hh][8 * g]);
-                o[et] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bh, o[et], 0, 0, 0);
-                o[et] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bl, o[et], 0, 0, 0);
+                o[et] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bp, o[et], 0, 0, 0);
             }
         }
     };
 
-    // Two register sets, alternating (no copies between them); past the
-    // wave's last tile the prefetch reloads that tile, unused. Loads retire
-    // in issue order, so the issue order is page(t + 2), data(t + 1), then
-    // tile t's products: each wait is for the oldest loads in flight only.
+    // Two register sets, alternating (no copies between them). Loads retire in issue
+    // order, so the issue order is pages(t + 2), data(t + 1), then tile t's products:
+    // each wait is for the oldest loads in flight only. q's loads go out behind the
+    // first pages and are converted while the first tiles' rows are on their way.
     if (ntile > 0 && ntile <= 4) {
         // splits of up to 512 keys: straight-line, every load unconditional
         // (only the products of tiles past the wave's last are skipped)
-        const int last = ntile - 1;
-        const int p0 = page_of(0), p1 = page_of(min(1, last));
-        Tile ta = load_tile(0, p0);
-        const int p2 = page_of(min(2, last));
+        const Pos x1 = next_pos(pos), x2 = next_pos(x1), x3 = next_pos(x2);
+        const int p0 = page_of(pos), p1 = page_of(x1), p2 = page_of(x2), p3 = page_of(x3);
         __builtin_amdgcn_sched_barrier(0);  // keep the issue order
-        Tile tb = load_tile(min(1, last), p1);
-        const int p3 = page_of(min(3, last));
+        load_q();
         __builtin_amdgcn_sched_barrier(0);
-        compute(ta);
-        ta = load_tile(min(2, last), p2);
+        Tile ta = load_tile(0, p0, pos);
         __builtin_amdgcn_sched_barrier(0);
-        if (ntile > 1) compute(tb);
-        tb = load_tile(min(3, last), p3);
+        Tile tb = load_tile(1, p1, x1);
         __builtin_amdgcn_sched_barrier(0);
-        if (ntile > 2) compute(ta);
-        if (ntile > 3) compute(tb);
+        prepare_q();
+        __builtin_amdgcn_sched_barrier(0);
+        compute(ta, true);
+        ta = load_tile(2, p2, x2);
+        __builtin_amdgcn_sched_barrier(0);
+        if (ntile > 1) compute(tb, false);
+        tb = load_tile(3, p3, x3);
+        __builtin_amdgcn_sched_barrier(0);
+        if (ntile > 2) compute(ta, false);
+        if (ntile > 3) compute(tb, false);
     } else if (ntile > 4) {
-        const int last = ntile - 1;
-        int pid_a = page_of(0);
-        int pid_b = page_of(min(1, last));
-        Tile ta = load_tile(0, pid_a), tb;
+        Pos xa = pos, xb = next_pos(pos);
+        int pid_a = page_of(xa), pid_b = page_of(xb);
+        __builtin_amdgcn_sched_barrier(0);
+        load_q();
+        __builtin_amdgcn_sched_barrier(0);
+        Tile ta = load_tile(0, pid_a, xa), tb;
+        __builtin_amdgcn_sched_barrier(0);
+        prepare_q();
+        __builtin_amdgcn_sched_barrier(0);
         for (int t = 0; t < ntile; t += 2) {
-            pid_a = page_of(min(t + 2, last));
+            xa = next_pos(xb);
+            pid_a = page_of(xa);
             __builtin_amdgcn_sched_barrier(0);
-            tb = load_tile(min(t + 1, last), pid_b);
+            tb = load_tile(t + 1, pid_b, xb);
             __builtin_amdgcn_sched_barrier(0);
-            compute(ta);
+            compute(ta, false);
             if (t + 1 >= ntile) break;
-            pid_b = page_of(min(t + 3, last));
+            xb = next_pos(xa);
+            pid_b = page_of(xb);
             __builtin_amdgcn_sched_barrier(0);
-            ta = load_tile(min(t + 2, last), pid_a);
+            ta = load_tile(t + 2, pid_a, xa);
             __builtin_amdgcn_sched_barrier(0);
-            compute(tb);
+            compute(tb, false);
         }
     }
 
-    // ---- merge the four waves (fixed order), then write
+    // ---- the two halves of O, then the four waves (fixed order), then write
+#pragma unroll
+    for (int et = 0; et < HD / 16; ++et)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[et][r] += other_half(o[et][r]);
     if (lane < 16) {
         lm[wave][lane] = m_run;
         ll[wave][lane] = l_run;
@@ -1382,7 +1459,7 @@ __global__ __launch_bounds__(256, 2) void vk_paged_attn_gqa(KvDev c, int layer, 
     float L = 0.0f;
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) L += ll[w][hh] * __expf(lm[w][hh] - M_use);
-    const float f = __expf(m_run - M_use);
+    const float f = __expf(m_run - M_use) * kVUnscale;
     vk_f32x4* red = reinterpret_cast<vk_f32x4*>(&lvt[0][0][0]);
     if (wave > 0) {
 #pragma unroll
