@@ -394,6 +394,17 @@ int run_gemm_qact(vokra_hip_ctx* c, const vokra_hip_qweight* w, const vokra_hip_
 
 int run_gemm(vokra_hip_ctx* c, const vokra_hip_qweight* w, size_t m, const float* d_a, const float* d_bias,
              float* d_out, int act_quant) {
+    // few rows on the decode kernel: the activation pass runs inside the linear, unless
+    // the output overlaps the rows that every workgroup reads
+    const bool apart = d_out + m * w->n <= d_a || d_a + m * w->k <= d_out;
+    if (!w->kquant && act_quant != VOKRA_HIP_ACT_KQUANT && w->has_gemv && c->decode_kernel && m <= kGemvMaxM && apart &&
+        vk::gemv_act_fits((int)m, (int)w->n, (int)w->nb)) {
+        const VkGemvLin lin = {(const uint4*)w->gq.p, (const uint2*)w->gsc.p, d_bias, d_out, {nullptr, 0}, (int)w->n};
+        VK_TRY(vk::launch_gemv_qblock_act(c->stream, wd_kv_mode(w->wdtype), act_quant == VOKRA_HIP_ACT_POW2, d_a, lin,
+                                          (int)m, (int)w->nb),
+               "launch(vk_gemv_qblock)");
+        return VOKRA_HIP_OK;
+    }
     int st = quantize_activations(c, &c->act, d_a, m, w->k, w->kquant ? VOKRA_HIP_ACT_KQUANT : act_quant);
     if (st) return st;
     return run_gemm_qact(c, w, &c->act, d_bias, d_out);

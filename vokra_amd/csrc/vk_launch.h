@@ -102,6 +102,9 @@ namespace vk {
 hipError_t launch_repack_w_gemv(hipStream_t s, int mode, const uint8_t* wq, int n, int n_pad, int nb, uint4* wq4,
                                 uint2* wsc);
 // n_lin (1..3) linears over the same activations, one launch.
+bool gemv_act_fits(int m, int n, int nb);
+hipError_t launch_gemv_qblock_act(hipStream_t s, int mode, bool pow2, const float* x, const VkGemvLin& lin, int m,
+                                  int nb);
 hipError_t launch_gemv_qblock(hipStream_t s, int mode, bool pow2, const uint4* afrag, const float* ascale,
                               const float* asum, const VkGemvLin* lins, int n_lin, int m, int nb, int m_pad);
 // One linear whose outputs feed the activation pass of the next input (qo:
