@@ -522,6 +522,206 @@ __global__ __launch_bounds__(64 * lg::WAVES) void vk_logits_argmax(const float* 
     }
 }
 
+// ---------------------------------------------------------------------------
+// The same for large vocabularies, f32 products on the bf16 matrix cores: every operand
+// is split exactly into three bf16 values, a = a0 + a1 + a2 (each the rounding of what the ones before leave),
+// and a . b is the sum of a0 b0, a0 b1, a1 b0, a1 b1, a0 b2 and a2 b0 in f32
+// accumulators. What is left out is below 2^-24 |a b|, the size of one rounding of an
+// f32 sum of the same terms; six v_mfma_f32_16x16x32_bf16 take 96 clocks per 32 k
+// where v_mfma_f32_16x16x4_f32 takes 256.
+// A finite operand that rounds to an infinite bf16, and operands that are not finite,
+// leave a logit that is not finite: those are computed again with f32 products.
+//
+// One workgroup per 128 vocabulary rows and up to 16 * NCT streams, k in steps of 32.
+// Vocabulary rows are on the 16-row side: a wave owns 32 of them and loads its own
+// fragments straight to registers (lane l holds k 8 (l / 16) .. +7 of row l % 16, whole
+// 128-byte lines), four steps ahead. The streams' fragments are shared: split by the
+// workgroup one step ahead into LDS, one barrier per step.
+//
+// Bound: memory, 4 bytes per weight: 64 streams, 51866 x 1280 (265 MB) 144
+// -> 86 us (52 at the rate of a copy, 30 of products and splits on each SIMD).
+// Error against 64 bits, relative to the largest logit: 1.6e-7, the f32 kernel's 5.2e-7.
+namespace lx3 {
+constexpr int WAVES = 4, RING = 4;  // RING: steps of vocabulary rows in flight
+static_assert(logits_d_multiple() % (32 * RING) == 0 && logits_min_d() >= 32 * RING, "whole rings");
+}  // namespace lx3
+
+// eight f32 values -> their three bf16 parts
+struct VkBf16x3 {
+    vk_bf16x8 p[3];
+};
+__device__ __forceinline__ VkBf16x3 vk_split_bf16x3(const float4& a, const float4& b) {
+    float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    VkBf16x3 r;
+#pragma unroll
+    for (int t = 0; t < 3; ++t)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            r.p[t][i] = (__bf16)v[i];
+            v[i] -= (float)r.p[t][i];
+        }
+    return r;
+}
+
+template <int NCT, int J, bool WRITE>
+__global__ __launch_bounds__(64 * lx3::WAVES, 2) void vk_logits_argmax_x3(const float* __restrict__ x, const float* __restrict__ emb,
+                                                              float* __restrict__ logits, float2* __restrict__ part,
+                                                              int n, int vocab, int d, int n_vt) {
+    using namespace lx3;
+    __shared__ __align__(16) uint4 lx[2][3][NCT][64];  // the streams' parts of a step, in fragment order
+    __shared__ float2 best[WAVES][16 * NCT];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int v0 = 16 * J * ((int)blockIdx.x * WAVES + wave), s0 = blockIdx.y * 16 * NCT;
+    const float4* ep[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+        ep[j] = reinterpret_cast<const float4*>(emb + (size_t)min(v0 + 16 * j + (lane & 15), vocab - 1) * d + 8 * (lane >> 4));
+    // staging: four threads hold a stream's 32 values of a step
+    const bool stage = tid < 64 * NCT;
+    const int ss = tid >> 2, sk = tid & 3;
+    const float4* xp = reinterpret_cast<const float4*>(x + (size_t)min(s0 + ss, n - 1) * d + 8 * sk);
+    uint4* xw = &lx[0][0][stage ? ss >> 4 : 0][(ss & 15) + 16 * sk];
+    constexpr int PART = NCT * 64, BUF = 3 * PART;
+    const int nk = d / 32;  // a multiple of RING
+    float4 er[RING][J][2], xr[2];
+    auto load_e = [&](int u, int ks) {
+        const int at = 8 * min(ks, nk - 1);  // past the end: the last step again, unused
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            er[u][j][0] = ep[j][at];
+            er[u][j][1] = ep[j][at + 1];
+        }
+    };
+    auto load_x = [&](int ks) {
+        const int at = 8 * min(ks, nk - 1);
+        if (stage) {
+            xr[0] = xp[at];
+            xr[1] = xp[at + 1];
+        }
+    };
+    auto store_x = [&](int buf) {
+        if (!stage) return;
+        const VkBf16x3 t = vk_split_bf16x3(xr[0], xr[1]);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) xw[buf * BUF + p * PART] = __builtin_bit_cast(uint4, t.p[p]);
+    };
+    // a0 b0 apart from the five smaller products, and summed over one ring at a time:
+    // the large sums round once per step, in short chains
+    vk_f32x4 acc[J][NCT], low[J][NCT];
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int c = 0; c < NCT; ++c) acc[j][c] = low[j][c] = {0.0f, 0.0f, 0.0f, 0.0f};
+    load_x(0);
+#pragma unroll
+    for (int u = 0; u < RING; ++u) load_e(u, u);
+    store_x(0);
+    load_x(1);
+    VK_LDS_BARRIER();
+#pragma unroll 1
+    for (int k0 = 0; k0 < nk; k0 += RING) {
+        vk_f32x4 top[J][NCT];
+#pragma unroll
+        for (int u = 0; u < RING; ++u) {
+            const int ks = k0 + u;
+            store_x((u + 1) & 1);  // step ks + 1 (past the end: unused)
+            load_x(ks + 2);
+            VkBf16x3 ea[J];
+#pragma unroll
+            for (int j = 0; j < J; ++j) ea[j] = vk_split_bf16x3(er[u][j][0], er[u][j][1]);
+            load_e(u, ks + RING);
+            // CG column tiles at a time: at least four independent chains between dependent products
+            constexpr int CG = NCT == 3 ? 3 : NCT * J > 4 ? 2 : NCT;
+#pragma unroll
+            for (int cg = 0; cg < NCT; cg += CG) {
+                vk_bf16x8 b[CG][3];
+#pragma unroll
+                for (int c = 0; c < CG; ++c)
+#pragma unroll
+                    for (int p = 0; p < 3; ++p) b[c][p] = __builtin_bit_cast(vk_bf16x8, lx[u & 1][p][cg + c][lane]);
+#pragma unroll
+                for (int t = 0; t < 6; ++t) {
+                    constexpr int PA[6] = {2, 0, 0, 1, 1, 0}, PB[6] = {0, 0, 2, 1, 0, 1};
+#pragma unroll
+                    for (int c = 0; c < CG; ++c)
+#pragma unroll
+                        for (int j = 0; j < J; ++j) {
+                            vk_f32x4& to = t == 1 ? top[j][cg + c] : low[j][cg + c];
+                            const vk_f32x4 from = t == 1 && u == 0 ? (vk_f32x4){0.0f, 0.0f, 0.0f, 0.0f} : to;
+                            to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ea[j].p[PA[t]], b[c][PB[t]], from, 0, 0, 0);
+                        }
+                }
+            }
+            VK_LDS_BARRIER();
+        }
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+#pragma unroll
+            for (int c = 0; c < NCT; ++c)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[j][c][r] += top[j][c][r];
+    }
+#pragma unroll
+    for (int c = 0; c < NCT; ++c) {
+        const int s = s0 + 16 * c + (lane & 15);
+        bool bad = false;
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                acc[j][c][r] += low[j][c][r];
+                bad |= !__builtin_isfinite(acc[j][c][r]);
+            }
+        if (__any(bad)) {  // f32 products, for the logits that are not finite
+            const float* xs = x + (size_t)min(s, n - 1) * d + 4 * (lane >> 4);
+#pragma unroll 1
+            for (int j = 0; j < J; ++j) {
+                const float* es = emb + (size_t)min(v0 + 16 * j + (lane & 15), vocab - 1) * d + 4 * (lane >> 4);
+                vk_f32x4 f = {0.0f, 0.0f, 0.0f, 0.0f};
+                for (int k = 0; k < d; k += 16) {
+                    const float4 a = *reinterpret_cast<const float4*>(es + k), b = *reinterpret_cast<const float4*>(xs + k);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        f = __builtin_amdgcn_mfma_f32_16x16x4f32(vk_f4c(a, i), vk_f4c(b, i), f, 0, 0, 0);
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    if (j == 0) acc[0][c][r] = __builtin_isfinite(acc[0][c][r]) ? acc[0][c][r] : f[r];
+                    else acc[J - 1][c][r] = __builtin_isfinite(acc[J - 1][c][r]) ? acc[J - 1][c][r] : f[r];
+                }
+            }
+        }
+        float bv = -INFINITY;
+        int bi = INT_MAX;
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int v = v0 + 16 * j + 4 * (lane >> 4) + r;  // ascending within the lane
+                if (v < vocab) {
+                    const float t = acc[j][c][r];
+                    if (WRITE && s < n) logits[(size_t)s * vocab + v] = t;
+                    if (t > bv) {
+                        bv = t;
+                        bi = v;
+                    }
+                }
+            }
+        // lanes l, l^16, l^32, l^48 hold the same stream
+        vk_am_merge(bv, bi, __shfl_xor(bv, 16, VK_WAVE), __shfl_xor(bi, 16, VK_WAVE));
+        vk_am_merge(bv, bi, __shfl_xor(bv, 32, VK_WAVE), __shfl_xor(bi, 32, VK_WAVE));
+        if (lane < 16) best[wave][16 * c + lane] = make_float2(bv, __int_as_float(bi));
+    }
+    __syncthreads();
+    if (tid < 16 * NCT && s0 + tid < n) {
+        float bv = best[0][tid].x;
+        int bi = __float_as_int(best[0][tid].y);
+#pragma unroll
+        for (int w = 1; w < WAVES; ++w) vk_am_merge(bv, bi, best[w][tid].x, __float_as_int(best[w][tid].y));
+        part[(size_t)(s0 + tid) * n_vt + blockIdx.x] = make_float2(bv, __int_as_float(bi));
+    }
+}
+
 // One workgroup per stream: merge its n_vt (max, index) partials. A partial
 // whose max is -inf holds no candidate; the result is index 0 when no value
 // beats -inf, as in the sampler.
@@ -695,6 +895,39 @@ static void go_logits(hipStream_t s, const float* x, const float* emb, float* lo
         hipLaunchKernelGGL((vk_logits_argmax<NCT, false>), grid, block, 0, s, x, emb, logits, part, n, vocab, d, n_vt);
 }
 
+template <int NCT, int J>
+static int go_logits_x3(hipStream_t s, const float* x, const float* emb, float* logits, float2* part, int n, int vocab,
+                     int d) {
+    const int n_vt = (vocab + 16 * J * lx3::WAVES - 1) / (16 * J * lx3::WAVES);
+    const dim3 grid((unsigned)n_vt, (unsigned)((n + 16 * NCT - 1) / (16 * NCT)));
+    const dim3 block(64 * lx3::WAVES);
+    if (logits)
+        hipLaunchKernelGGL((vk_logits_argmax_x3<NCT, J, true>), grid, block, 0, s, x, emb, logits, part, n, vocab, d, n_vt);
+    else
+        hipLaunchKernelGGL((vk_logits_argmax_x3<NCT, J, false>), grid, block, 0, s, x, emb, logits, part, n, vocab, d, n_vt);
+    return n_vt;
+}
+
+// A 16-row tile more per wave halves the reads of the streams per weight, where it
+// does not leave a CU with more rows than the finer split (64 streams, k 1280, us, 1 /
+// 2 tiles: 51866 rows 105 / 86, 40000 66 / 73, 20000 50 / 54).
+template <int NCT>
+static int go_logits_wide(hipStream_t s, const float* x, const float* emb, float* logits, float2* part, int n, int vocab,
+                          int d) {
+    const int wg1 = (vocab + 63) / 64, wg2 = (vocab + 127) / 128;
+    return wg2 > 256 && (wg2 + 255) / 256 * 2 <= (wg1 + 255) / 256
+               ? go_logits_x3<NCT, 2>(s, x, emb, logits, part, n, vocab, d)
+               : go_logits_x3<NCT, 1>(s, x, emb, logits, part, n, vocab, d);
+}
+
+// Vocabularies from which the three-part kernel runs, whatever the number of streams (a
+// stream's logits do not depend on its batch): its k loop is one chain per workgroup,
+// four times as long as the f32 kernel's, and needs about two workgroups per CU to hide
+// it. f32 / three-part, us: 51866 x 1280: 64 streams 144 / 86, 17 71 / 58, 16 65 / 54, 8
+// 58 / 53, 1 50 / 54; 40000 x 1280, 64 streams 93 / 66; 32000 x 2048 115 / 84; 20000 x
+// 1280: 64 streams 57 / 50, 16 29 / 31; 5000 x 512, 64 streams 14.5 / 19.
+constexpr int kLogitsWideFrom = 30720;
+
 hipError_t launch_logits_argmax(hipStream_t s, const float* x, const float* emb, float* logits, float2* part,
                                 int* next, int n, int vocab, int d) {
     if (n == 0) return hipSuccess;
@@ -703,9 +936,14 @@ hipError_t launch_logits_argmax(hipStream_t s, const float* x, const float* emb,
     if (vocab < 1 || d < logits_min_d() || d % logits_d_multiple() != 0) return hipErrorInvalidValue;
     // whole chunks per wave, and enough of them to fill the ring
     if (d % (16 * lg::WAVES) != 0 || d / (16 * lg::WAVES) < lg::NSLOT - 1) return hipErrorInvalidValue;
-    const int n_vt = logits_n_vt(vocab);
     if ((n + 63) / 64 > 65535) return hipErrorInvalidValue;  // grid.y limit
-    if (n <= 16) go_logits<1>(s, x, emb, logits, part, n, vocab, d, n_vt);
+    int n_vt = logits_n_vt(vocab);
+    if (vocab >= kLogitsWideFrom) {
+        if (n <= 16) n_vt = go_logits_wide<1>(s, x, emb, logits, part, n, vocab, d);
+        else if (n <= 32) n_vt = go_logits_wide<2>(s, x, emb, logits, part, n, vocab, d);
+        else if (n <= 48) n_vt = go_logits_wide<3>(s, x, emb, logits, part, n, vocab, d);
+        else n_vt = go_logits_wide<4>(s, x, emb, logits, part, n, vocab, d);
+    } else if (n <= 16) go_logits<1>(s, x, emb, logits, part, n, vocab, d, n_vt);
     else if (n <= 32) go_logits<2>(s, x, emb, logits, part, n, vocab, d, n_vt);
     else if (n <= 48) go_logits<3>(s, x, emb, logits, part, n, vocab, d, n_vt);
     else go_logits<4>(s, x, emb, logits, part, n, vocab, d, n_vt);
