@@ -546,23 +546,25 @@ constexpr int WAVES = 4, RING = 4;  // RING: steps of vocabulary rows in flight
 static_assert(logits_d_multiple() % (32 * RING) == 0 && logits_min_d() >= 32 * RING, "whole rings");
 }  // namespace lx3
 
-// eight f32 values -> their three bf16 parts
+// W f32 values -> their three bf16 parts
+template <int W>
 struct VkBf16x3 {
-    vk_bf16x8 p[3];
+    __bf16 __attribute__((ext_vector_type(W))) p[3];
 };
-__device__ __forceinline__ VkBf16x3 vk_split_bf16x3(const float4& a, const float4& b) {
-    float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-    VkBf16x3 r;
+template <int W>
+__device__ __forceinline__ VkBf16x3<W> vk_split_bf16x3(float __attribute__((ext_vector_type(W))) v) {
+    VkBf16x3<W> r;
 #pragma unroll
     for (int t = 0; t < 3; ++t)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < W; ++i) {
             r.p[t][i] = (__bf16)v[i];
             v[i] -= (float)r.p[t][i];
         }
     return r;
 }
 
+using vk_f32x8 = float __attribute__((ext_vector_type(8)));
 template <int NCT, int J, bool WRITE>
 __global__ __launch_bounds__(64 * lx3::WAVES, 2) void vk_logits_argmax_x3(const float* __restrict__ x, const float* __restrict__ emb,
                                                               float* __restrict__ logits, float2* __restrict__ part,
@@ -576,34 +578,33 @@ __global__ __launch_bounds__(64 * lx3::WAVES, 2) void vk_logits_argmax_x3(const 
 #pragma unroll
     for (int j = 0; j < J; ++j)
         ep[j] = reinterpret_cast<const float4*>(emb + (size_t)min(v0 + 16 * j + (lane & 15), vocab - 1) * d + 8 * (lane >> 4));
-    // staging: four threads hold a stream's 32 values of a step
-    const bool stage = tid < 64 * NCT;
-    const int ss = tid >> 2, sk = tid & 3;
-    const float4* xp = reinterpret_cast<const float4*>(x + (size_t)min(s0 + ss, n - 1) * d + 8 * sk);
-    uint4* xw = &lx[0][0][stage ? ss >> 4 : 0][(ss & 15) + 16 * sk];
-    constexpr int PART = NCT * 64, BUF = 3 * PART;
+    // staging: 32 / XW threads hold a stream's 32 values of a step (with three column tiles a
+    // quarter of the threads load a copy, unused)
+    constexpr int XW = NCT == 1 ? 2 : NCT == 2 ? 4 : 8;
+    using XVec = float __attribute__((ext_vector_type(XW)));
+    const int ss = tid / (32 / XW), sk = XW * (tid % (32 / XW));
+    const bool stage = ss < 16 * NCT;
+    const float* xp = x + (size_t)min(s0 + (stage ? ss : 0), n - 1) * d + sk;
+    char* xw = reinterpret_cast<char*>(&lx[0][0][stage ? ss >> 4 : 0][(ss & 15) + 16 * (sk >> 3)]) + 2 * (sk & 7);
+    constexpr int PART = NCT * 64 * 16, BUF = 3 * PART;  // bytes
     const int nk = d / 32;  // a multiple of RING
-    float4 er[RING][J][2], xr[2];
+    vk_f32x8 er[RING][J];
+    XVec xr[RING];
     auto load_e = [&](int u, int ks) {
         const int at = 8 * min(ks, nk - 1);  // past the end: the last step again, unused
 #pragma unroll
         for (int j = 0; j < J; ++j) {
-            er[u][j][0] = ep[j][at];
-            er[u][j][1] = ep[j][at + 1];
+            const float4 a = ep[j][at], b = ep[j][at + 1];
+            er[u][j] = (vk_f32x8){a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
         }
     };
-    auto load_x = [&](int ks) {
-        const int at = 8 * min(ks, nk - 1);
-        if (stage) {
-            xr[0] = xp[at];
-            xr[1] = xp[at + 1];
-        }
-    };
-    auto store_x = [&](int buf) {
+    auto load_x = [&](int u, int ks) { __builtin_memcpy(&xr[u], __builtin_assume_aligned(xp + 32 * min(ks, nk - 1), XW == 2 ? 8 : 16), 4 * XW); };
+    auto store_x = [&](int u, int buf) {
+        const VkBf16x3<XW> t = vk_split_bf16x3<XW>(xr[u]);
         if (!stage) return;
-        const VkBf16x3 t = vk_split_bf16x3(xr[0], xr[1]);
 #pragma unroll
-        for (int p = 0; p < 3; ++p) xw[buf * BUF + p * PART] = __builtin_bit_cast(uint4, t.p[p]);
+        for (int p = 0; p < 3; ++p)
+            __builtin_memcpy(__builtin_assume_aligned(xw + buf * BUF + p * PART, 2 * XW), &t.p[p], 2 * XW);
     };
     // a0 b0 apart from the five smaller products, and summed over one ring at a time:
     // the large sums round once per step, in short chains
@@ -612,11 +613,14 @@ __global__ __launch_bounds__(64 * lx3::WAVES, 2) void vk_logits_argmax_x3(const 
     for (int j = 0; j < J; ++j)
 #pragma unroll
         for (int c = 0; c < NCT; ++c) acc[j][c] = low[j][c] = {0.0f, 0.0f, 0.0f, 0.0f};
-    load_x(0);
+    load_x(0, 0);
 #pragma unroll
-    for (int u = 0; u < RING; ++u) load_e(u, u);
-    store_x(0);
-    load_x(1);
+    for (int u = 0; u < RING; ++u) {
+        if (u + 1 < RING) load_x(u + 1, u + 1);
+        load_e(u, u);
+    }
+    store_x(0, 0);
+    load_x(0, RING);
     VK_LDS_BARRIER();
 #pragma unroll 1
     for (int k0 = 0; k0 < nk; k0 += RING) {
@@ -624,11 +628,11 @@ __global__ __launch_bounds__(64 * lx3::WAVES, 2) void vk_logits_argmax_x3(const 
 #pragma unroll
         for (int u = 0; u < RING; ++u) {
             const int ks = k0 + u;
-            store_x((u + 1) & 1);  // step ks + 1 (past the end: unused)
-            load_x(ks + 2);
-            VkBf16x3 ea[J];
+            store_x((u + 1) % RING, (u + 1) & 1);  // step ks + 1 (past the end: unused)
+            load_x((u + 1) % RING, ks + 1 + RING);
+            VkBf16x3<8> ea[J];
 #pragma unroll
-            for (int j = 0; j < J; ++j) ea[j] = vk_split_bf16x3(er[u][j][0], er[u][j][1]);
+            for (int j = 0; j < J; ++j) ea[j] = vk_split_bf16x3<8>(er[u][j]);
             load_e(u, ks + RING);
             // CG column tiles at a time: at least four independent chains between dependent products
             constexpr int CG = NCT == 3 ? 3 : NCT * J > 4 ? 2 : NCT;
