@@ -1035,13 +1035,16 @@ __global__ __launch_bounds__(256, 5) void vk_paged_attn_w64(KvDev c, int layer, 
 //     K quants are exact fp16 integers, so each block dot is the exact integer
 //     dot against the two fp16 halves of q * scale; the key's f16 block scale
 //     is applied to the block sum (v_mfma_f32_16x16x32_f16, keys on the 16-row
-//     side, heads on the 16-column side);
+//     side, heads on the 16-column side, padded to 16);
 //   O^T[dim][head] += V^T . (p * d_v)^T
 //     the V block scale of each key folds into P, split hi/lo; V^T comes from
 //     a per-wave LDS copy of the tile converted to fp16.
-// With at most 8 heads the halves share one product: column h holds head h's hi
-// half and column h + 8 its lo half, and the two columns are added where a result
-// is needed (S per tile, O once), so both columns of a head carry the same softmax.
+// The hi and the lo half of an operand go through one accumulator, hi first: a block
+// dot is rounded as a whole before its scale is applied. (The halves in columns h and
+// h + 8 of one product save a matrix instruction per block, but each half is then
+// scaled and summed by itself: other last bits, which the INT8 activations behind the
+// attention carry on as whole steps; and no time: four layers of 32 items, 512 .. 4096
+// keys, 132.5 us with one product, 132.8 with two.)
 //
 // Each wave owns the 32-key tiles j0 = k0 + 32 w + 128 i of the split and keeps
 // its own online softmax; the four states merge in wave order at the end.
@@ -1101,7 +1104,7 @@ __global__ __launch_bounds__(256, 2) void vk_paged_attn_gqa(KvDev c, int layer, 
                                                          const float* __restrict__ ak, const float* __restrict__ av,
                                                          const int* __restrict__ at) {
     using namespace pg;
-    static_assert(G >= 2 && G <= 8, "query heads per kv head: their two halves fill the 16 columns");
+    static_assert(G >= 2 && G <= 16, "query heads per kv head: one per column");
     __shared__ __align__(16) _Float16 lvt[WAVES][HD][VROW];  // per wave: V^T of its tile (reused by the merge)
     __shared__ float lm[WAVES][16], ll[WAVES][16];
     static_assert(sizeof(lvt) >= sizeof(vk_f32x4) * (WAVES - 1) * (HD / 16) * 64, "merge buffer fits");
@@ -1152,13 +1155,11 @@ __global__ __launch_bounds__(256, 2) void vk_paged_attn_gqa(KvDev c, int layer, 
         }
     }
 
-    // q * scale of the column's head (zero for padding heads) as the S^T B operand:
-    // lane (g, hh) holds dims 32b + 8g .. +7 of head hh % 8, the fp16 hi half in
-    // columns 0..7 and the lo half in columns 8..15. With rope_cs, q is first
+    // q * scale of head hh (zero for padding heads) as the S^T B operand: lane (g, hh)
+    // holds dims 32b + 8g .. +7, split into fp16 hi + lo. With rope_cs, q is first
     // rotated: dims j and j + 64 (blocks b and b + 2) sit in the same lane.
-    vk_h16x8_t qh[NB];
-    const float lo_mask = hh >= 8 ? -1.0f : 0.0f;  // part = x + mask * hi: x itself, or what hi leaves of it
-    const int qhead = min(hh & 7, G - 1);  // padding heads load the last one, unused
+    vk_h16x8_t qh[NB], ql[NB];
+    const int qhead = min(hh, G - 1);  // padding heads load the last one, unused
     float4 xq[NB][2], cs4[2][4];
     auto load_q = [&]() {
         const float4* qp = reinterpret_cast<const float4*>(q + ((size_t)item * hq + hk * G + qhead) * HD + 8 * g);
@@ -1198,13 +1199,12 @@ __global__ __launch_bounds__(256, 2) void vk_paged_attn_gqa(KvDev c, int layer, 
         for (int b = 0; b < NB; ++b)
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                float xs = (hh & 7) < G ? x[b][i] * scale : 0.0f;
+                float xs = hh < G ? x[b][i] * scale : 0.0f;
                 asm("" : "+v"(xs));  // see the P operand below
                 bad |= vk_f16_overflow(xs);
                 const _Float16 h = (_Float16)xs;
-                float part = fmaf((float)h, lo_mask, xs);
-                asm("" : "+v"(part));
-                qh[b][i] = (_Float16)part;
+                qh[b][i] = h;
+                ql[b][i] = (_Float16)(xs - (float)h);
             }
         if (bad) atomicOr(&vk_kv_range_flag, 1u);
     };
@@ -1281,10 +1281,6 @@ __global__ __launch_bounds__(256, 2) void vk_paged_attn_gqa(KvDev c, int layer, 
         }
         return T;
     };
-    // the value of the other column of this head (hi <-> lo): DPP row_ror 8
-    auto other_half = [](float v) {
-        return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x128, 0xf, 0xf, true));
-    };
     auto compute = [&](const Tile& T, bool first) {
         // scales of keys 8g + j (j = 4n + r) from the lanes that loaded them
         uint2 kds[8], vds[8];
@@ -1304,6 +1300,7 @@ __global__ __launch_bounds__(256, 2) void vk_paged_attn_gqa(KvDev c, int layer, 
                 const vk_h16x8_t a = vk_i8x8_f16(T.kw[n][b]);
                 vk_f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
                 d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qh[b], d, 0, 0, 0);
+                d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, ql[b], d, 0, 0, 0);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const vk_h16x2_t kd = __builtin_bit_cast(vk_h16x2_t, b < 2 ? kds[4 * n + r].x : kds[4 * n + r].y);
@@ -1311,7 +1308,7 @@ __global__ __launch_bounds__(256, 2) void vk_paged_attn_gqa(KvDev c, int layer, 
                 }
             }
 #pragma unroll
-            for (int r = 0; r < 4; ++r) sc[4 * n + r] = acc[r] + other_half(acc[r]);
+            for (int r = 0; r < 4; ++r) sc[4 * n + r] = acc[r];
         }
         if (!__all(T.has)) {  // keys past the split or without a page
 #define VK_GQA_HAS(J) sc[J] = vk_row_bcast_i<J>(T.has) ? sc[J] : -INFINITY;
@@ -1367,24 +1364,25 @@ __global__ __launch_bounds__(256, 2) void vk_paged_attn_gqa(KvDev c, int layer, 
         // ---- O^T += V^T . (p d_v)^T, one V block scale per pair of 16-dim tiles
 #pragma unroll
         for (int vb = 0; vb < NB; ++vb) {
-            vk_h16x8_t bp;  // hi, or lo = pd - hi: the mask keeps it branchless
+            vk_h16x8_t bh, bl;
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const vk_h16x2_t d2 = __builtin_bit_cast(vk_h16x2_t, vb < 2 ? vds[j].x : vds[j].y);
                 float pd = fmaf(p[j], (float)d2[vb & 1], zero);  // the product, with the scale taken as fp16
-                // both columns must split the same f32 value: a conversion fused into
-                // the operation before it rounds once where the other column rounds
+                // both halves must split the same f32 value: a conversion fused into the
+                // operation before it rounds once where the subtraction's operand rounds
                 // twice, and hi + lo is then off by an fp16 ulp of hi
                 asm("" : "+v"(pd));
-                float part = fmaf((float)(_Float16)pd, lo_mask, pd);
-                asm("" : "+v"(part));
-                bp[j] = (_Float16)part;
+                const _Float16 h = (_Float16)pd;
+                bh[j] = h;
+                bl[j] = (_Float16)(pd - (float)h);
             }
 #pragma unroll
             for (int e2 = 0; e2 < 2; ++e2) {
                 const int et = 2 * vb + e2;
                 const vk_h16x8_t a = *reinterpret_cast<const vk_h16x8_t*>(&lvt[wave][16 * et + hh][8 * g]);
-                o[et] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bp, o[et], 0, 0, 0);
+                o[et] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bh, o[et], 0, 0, 0);
+                o[et] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bl, o[et], 0, 0, 0);
             }
         }
     };
@@ -1442,11 +1440,7 @@ __global__ __launch_bounds__(256, 2) void vk_paged_attn_gqa(KvDev c, int layer, 
         }
     }
 
-    // ---- the two halves of O, then the four waves (fixed order), then write
-#pragma unroll
-    for (int et = 0; et < HD / 16; ++et)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[et][r] += other_half(o[et][r]);
+    // ---- merge the four waves (fixed order), then write
     if (lane < 16) {
         lm[wave][lane] = m_run;
         ll[wave][lane] = l_run;
