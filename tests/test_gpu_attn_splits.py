@@ -2,9 +2,12 @@
 tiles and heads, several key tiles) and of their merge, against float64, at the
 edges of tiles and chunks; an item alone equals the item in a batch, both in one
 that splits and in one that runs the chunks in place, bit for bit."""
+import ctypes
+
 import numpy as np
 import pytest
 
+from tests.test_gpu_sessions import enc_layer
 from vokra_amd import hip
 
 pytestmark = pytest.mark.gpu
@@ -52,7 +55,10 @@ def test_key_splits_vs_float64(ctx, hd, hq, hkv, tq, tkv, causal):
     assert np.abs(got - want).max() <= 2e-5
 
 
-@pytest.mark.parametrize("hd,hq,hkv,t,batch", [(64, 8, 8, 700, 2), (64, 8, 8, 700, 9), (128, 8, 2, 300, 3)])
+# over workgroups in one launch, in place at both head_dims (768 query tiles and heads
+# or more), and over workgroups in slices of the batch
+@pytest.mark.parametrize("hd,hq,hkv,t,batch", [(64, 8, 8, 700, 2), (64, 8, 8, 700, 9), (128, 8, 2, 300, 3),
+                                               (128, 16, 2, 300, 10), (64, 1, 1, 704, 60)])
 def test_split_item_does_not_depend_on_the_batch(ctx, hd, hq, hkv, t, batch):
     print(f"[case] split attention batch {batch} == alone, hd {hd}", flush=True)
     g = np.random.default_rng(batch)
@@ -74,3 +80,90 @@ def test_non_finite_values_stay_in_their_rows(ctx):
     v[0, 600, 5] = np.nan
     got = ctx.attn_f32(q, k, v, H, causal=False)[0]
     assert np.isnan(got[:, 5]).all() and np.isnan(got).sum() == t
+
+
+class At:
+    """A device buffer's pointer, `off` bytes in."""
+
+    def __init__(self, buf, off):
+        self.buf, self.ptr = buf, ctypes.c_void_p(buf.ptr.value + off)
+
+
+def test_slices_of_a_batch_equal_its_items(ctx):
+    """Few queries over many keys: more chunks than the partials' workspace holds."""
+    g = np.random.default_rng(4)
+    batch, tq, tkv, hd = 700, 3, 704, 64
+    q = g.standard_normal((batch, tq, hd)).astype(np.float32)
+    k = g.standard_normal((batch, tkv, hd)).astype(np.float32)
+    v = g.standard_normal((batch, tkv, hd)).astype(np.float32)
+    full = ctx.attn_f32(q, k, v, 1)
+    for b in (0, 681, 682, 683, batch - 1):
+        assert np.array_equal(ctx.attn_f32(q[b], k[b], v[b], 1), full[b])
+
+
+@pytest.mark.parametrize("hd,h,t", [(64, 4, 321), (128, 2, 130)])
+def test_values_off_16_bytes(ctx, hd, h, t):
+    """v may start anywhere (q, k and out are 16-byte aligned)."""
+    g = np.random.default_rng(hd)
+    q, k, v = (g.standard_normal((t, h * hd)).astype(np.float32) for _ in range(3))
+    want = ctx.attn_f32(q, k, v, h)
+    d_q, d_k = (hip.DeviceBuffer.from_array(ctx, x) for x in (q, k))
+    d_v = hip.DeviceBuffer.from_array(ctx, np.concatenate([np.full(1, 9.0, np.float32), v.reshape(-1)]))
+    d_o = hip.DeviceBuffer(ctx, q.nbytes)
+    ctx.attn_f32_dev(1, t, t, h, h, hd, d_q, d_k, At(d_v, 4), hd ** -0.5, False, 0, d_o)
+    ctx.synchronize()
+    assert np.array_equal(d_o.download(np.float32, q.size).reshape(q.shape), want)
+
+
+def test_captured_split_without_its_workspace():
+    """A capture on a context whose calls have not split their keys yet allocates
+    nothing and replays the eager call's bits."""
+    ctx = hip.HipContext(0)
+    g = np.random.default_rng(11)
+    wide = [hip.DeviceBuffer.from_array(ctx, g.standard_normal((800, 40 * 64)).astype(np.float32)) for _ in range(4)]
+    ctx.attn_f32_dev(1, 800, 800, 40, 40, 64, *wide[:3], 0.125, False, 0, wide[3])  # 520 query tiles and heads: whole
+    q, k, v = (g.standard_normal((1500, 8 * 64)).astype(np.float32) for _ in range(3))
+    d = [hip.DeviceBuffer.from_array(ctx, x) for x in (q, k, v)]
+    d_o = hip.DeviceBuffer(ctx, q.nbytes)
+    graph = ctx.capture(lambda: ctx.attn_f32_dev(1, 1500, 1500, 8, 8, 64, *d, 0.125, False, 0, d_o))
+    graph.launch()
+    ctx.synchronize()
+    first = d_o.download(np.float32, q.size)
+    ctx.attn_f32_dev(1, 1500, 1500, 8, 8, 64, *d, 0.125, False, 0, d_o)  # eager: over workgroups
+    ctx.synchronize()
+    want = d_o.download(np.float32, q.size)
+    assert np.array_equal(first, want)
+    for _ in range(2):
+        d_o.upload(np.zeros_like(q))
+        graph.launch()
+        ctx.synchronize()
+        assert np.array_equal(d_o.download(np.float32, q.size), want)
+    del graph
+    ctx.close()
+
+
+def test_captured_encoder_outlives_larger_attention_calls():
+    """A captured encoder forward whose attention splits its keys, replayed after eager
+    attention calls that split more: the partials' block is never replaced."""
+    ctx = hip.HipContext(0)
+    g = np.random.default_rng(12)
+    d, frames = 512, 700
+    layers = [enc_layer(ctx, g, hip.WDtype.Q8_0, d, 4 * d, scale=0.02)]
+    one, zero = np.ones(d, np.float32), np.zeros(d, np.float32)
+    enc = hip.Encoder(ctx, hip.WDtype.Q8_0, d, d // 64, 4 * d, layers, one, zero, frames)
+    x = g.standard_normal((1, frames, d)).astype(np.float32)
+    d_x, d_o = hip.DeviceBuffer.from_array(ctx, x), hip.DeviceBuffer(ctx, x.nbytes)
+    enc.forward_dev(1, frames, d_x, d_o)
+    ctx.synchronize()
+    want = d_o.download(np.float32, x.size)
+    graph = ctx.capture(lambda: enc.forward_dev(1, frames, d_x, d_o))
+    q, k, v = (g.standard_normal((777, 16 * 128)).astype(np.float32) for _ in range(3))
+    other = ctx.attn_f32(q, k, v, 16, causal=True)
+    for _ in range(3):
+        d_o.upload(np.zeros_like(x))
+        graph.launch()
+        ctx.synchronize()
+        assert np.array_equal(d_o.download(np.float32, x.size), want)
+        assert np.array_equal(ctx.attn_f32(q, k, v, 16, causal=True), other)
+    del graph, enc
+    ctx.close()

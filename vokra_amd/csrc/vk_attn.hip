@@ -343,7 +343,8 @@ __global__ __launch_bounds__(256) void vk_split_vt_q7(const float* __restrict__ 
 // (kl, vtl as fp16 arrays), 2 compact (one byte per element, split_q7).
 // SEQ: the key chunks of sp one after the other in this workgroup, each with a
 // softmax of its own, merged as vk_attn_combine merges them: the results of a
-// launch over chunks without its partials, for batches that fill the chip.
+// launch over chunks without its partials, for batches that fill the chip and for calls
+// that have no room for partials.
 template <int HD, int LOM, bool ONEQ, bool SEQ = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void vk_flash_attn(
     const uint4* __restrict__ qh, const uint4* __restrict__ ql,    // [B][Tq][Hq*HD] fp16, scaled
@@ -670,15 +671,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void v
     // SEQ: the chunks merged so far
     vk_f32x4 o_sum[SEQ ? OS : 1];
     float m_sum = -INFINITY, l_sum = 0.0f;
-    int chunk_left = sp.chunk;  // tiles of this chunk (SEQ)
-    bool merged = false;
-    auto merge = [&]() __attribute__((always_inline)) {
-        if (!merged) {
+    auto merge = [&](bool first) __attribute__((always_inline)) {
+        if (first) {
 #pragma unroll
             for (int os = 0; os < (SEQ ? OS : 1); ++os) o_sum[os] = o_acc[os];
             m_sum = m_run;
             l_sum = l_run;
-            merged = true;
         } else {
             const float mn = fmaxf(m_sum, m_run), mu = mn == -INFINITY ? 0.0f : mn;
             const float wa = __builtin_amdgcn_exp2f(m_sum - mu), wb = __builtin_amdgcn_exp2f(m_run - mu);
@@ -693,7 +691,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void v
         for (int os = 0; os < OS; ++os) o_acc[os] = {0.0f, 0.0f, 0.0f, 0.0f};
         m_run = -INFINITY;
         l_run = 0.0f;
-        chunk_left = sp.chunk;
     };
     Stage st = load(kt_first);  // unconditional (clamped) loads keep the stage in registers
     auto step = [&](int kt, auto mask_tag) __attribute__((always_inline)) {
@@ -701,19 +698,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void v
         st = load(min(kt + 1, n_tiles - 1));
         if (active) tile(kt, mask_tag);
         VK_LDS_BARRIER();
-        if constexpr (SEQ) {
-            if (--chunk_left == 0 || kt + 1 == n_tiles) merge();  // uniform
-        }
     };
     int n_full = min(n_tiles, tkv / KT);
     if (causal) n_full = min(n_full, (q_off + qt * QT + 1) / KT);
     int kt = kt_first;
-    for (; kt < n_full; ++kt) step(kt, AttnMask<false>{});
-    for (; kt < n_tiles; ++kt) step(kt, AttnMask<true>{});
     if constexpr (SEQ) {
+        for (int c0 = 0; c0 < n_tiles; c0 += sp.chunk) {
+            const int end = min(c0 + sp.chunk, n_tiles), full = min(end, n_full);
+            for (; kt < full; ++kt) step(kt, AttnMask<false>{});
+            for (; kt < end; ++kt) step(kt, AttnMask<true>{});
+            merge(c0 == 0);
+        }
         finish(o_sum, l_sum > 0.0f ? 1.0f / l_sum : 0.0f);
         return;
     }
+    for (; kt < n_full; ++kt) step(kt, AttnMask<false>{});
+    for (; kt < n_tiles; ++kt) step(kt, AttnMask<true>{});
     if constexpr (!ONEQ && !SEQ) {
         if (partial) {  // this chunk's (max, sum) and unscaled O; vk_attn_combine merges the chunks
             const size_t pid = (((size_t)b * hq + h) * gridDim.x + qt) * sp.n_split + chunk_i;
@@ -896,7 +896,7 @@ int oneq_lds_pad(int r_full, int lds_static, size_t n_wg) {
     return total > attn::kLdsPerCu / r_full && total > lds_static ? total - lds_static : 0;
 }
 
-template <int HD, int LOM, bool ONEQ>
+template <int HD, int LOM, bool ONEQ, bool SEQ = false>
 void go_flash(hipStream_t s, dim3 grid, const FlashArgs& a) {
     int pad = 0;
     if (ONEQ) {
@@ -910,16 +910,18 @@ void go_flash(hipStream_t s, dim3 grid, const FlashArgs& a) {
         pad = oneq_lds_pad(r_full, attn::flash_lds_bytes(HD, LOM != 0 ? 2 : 1),
                            (size_t)grid.x * grid.y * grid.z);
     }
-    hipLaunchKernelGGL((vk_flash_attn<HD, LOM, ONEQ>), grid, dim3(256), pad, s, (const uint4*)a.qh,
+    hipLaunchKernelGGL((vk_flash_attn<HD, LOM, ONEQ, SEQ>), grid, dim3(256), pad, s, (const uint4*)a.qh,
                        (const uint4*)a.ql, (const uint4*)a.kh, (const uint4*)a.kl, (const uint4*)a.vth,
                        (const uint4*)a.vtl, a.out, a.tq, a.tkv, a.t_pad, a.hq, a.hkv, a.causal, a.q_off, a.kv_index,
                        a.qf, a.q_scale, a.qo, a.lay, a.sp);
 }
 
 template <int HD>
-void go_flash_hd(hipStream_t s, dim3 grid, int lo_mode, const FlashArgs& a) {
+void go_flash_hd(hipStream_t s, dim3 grid, int lo_mode, const FlashArgs& a, bool seq) {
     const bool one = a.tq == 1;
-    if (lo_mode == KV_LO_Q7)  // the compact form exists for single-query launches only
+    if (seq)  // several queries with fp16 low parts only
+        go_flash<HD, 1, false, true>(s, grid, a);
+    else if (lo_mode == KV_LO_Q7)  // the compact form exists for single-query launches only
         go_flash<HD, 2, true>(s, grid, a);
     else if (lo_mode == KV_LO_F16)
         one ? go_flash<HD, 1, true>(s, grid, a) : go_flash<HD, 1, false>(s, grid, a);
@@ -927,17 +929,18 @@ void go_flash_hd(hipStream_t s, dim3 grid, int lo_mode, const FlashArgs& a) {
         one ? go_flash<HD, 0, true>(s, grid, a) : go_flash<HD, 0, false>(s, grid, a);
 }
 
-hipError_t flash_any(hipStream_t s, int hd, int batch, int lo_mode, const FlashArgs& a) {
+// seq: the chunks of a.sp inside each workgroup
+hipError_t flash_any(hipStream_t s, int hd, int batch, int lo_mode, const FlashArgs& a, bool seq = false) {
     if (lo_mode == KV_LO_Q7 && a.tq != 1) return hipErrorInvalidValue;
     // buffer-resource extents (one kv head's V^T slab, 64 K rows) and the
     // per-lane 32-bit K offsets, in bytes
     if ((size_t)hd * a.t_pad * 2 > 0x7fffffffu || (size_t)attn::KT * a.lay.kt * 2 > 0x7fffffffu)
         return hipErrorInvalidValue;
-    const dim3 grid((a.tq + attn::QT - 1) / attn::QT, a.hq, batch * a.sp.n_split);
+    const dim3 grid((a.tq + attn::QT - 1) / attn::QT, a.hq, seq ? batch : batch * a.sp.n_split);
     if (hd == 64)
-        go_flash_hd<64>(s, grid, lo_mode, a);
+        go_flash_hd<64>(s, grid, lo_mode, a, seq);
     else
-        go_flash_hd<128>(s, grid, lo_mode, a);
+        go_flash_hd<128>(s, grid, lo_mode, a, seq);
     return hipGetLastError();
 }
 }  // namespace
@@ -972,7 +975,7 @@ hipError_t launch_flash_attn_f32q(hipStream_t s, int hd, const float* q, float q
 // tiles, cross-attention with few queries, a few heads.
 // Measured (whole calls, us, before -> after): 1 x 777 causal, 16 / 2 heads x 128 48.4
 // -> 33.3; 1 x 1500, 8 heads x 64 51 -> 38; 16 queries over 1500 keys, 20 heads 51 ->
-// 22; 64 causal after 300, 32 / 8 x 128 29 -> 20; 8 x 1500, 8 heads (in place) 158 -> 163
+// 22; 64 causal after 300, 32 / 8 x 128 29 -> 20.
 constexpr long long kSplitTarget = 480;
 int attn_key_splits(int tq, int tkv, int hq, int causal, int q_off, int* chunk) {
     *chunk = 0;
@@ -995,42 +998,67 @@ int attn_key_splits(int tq, int tkv, int hq, int causal, int q_off, int* chunk) 
     return (int)n;
 }
 
-// Whether a batch's chunks run inside one workgroup per query tile instead
-// (SEQ; head_dim 64, where the merged state fits the registers): from one and a
-// half rounds of two workgroups per CU on, the chip is full without the split.
-bool attn_split_in_place(int hd, int batch, int tq, int hq) {
-    return hd == 64 && (long long)batch * hq * ((tq + attn::QT - 1) / attn::QT) >= 768;
+// Whether a batch's chunks run inside one workgroup per query tile instead (SEQ):
+// from one and a half rounds of two workgroups per CU on, the chip is full without
+// the split. Whole calls, us, undivided / in place / over workgroups: 8 x 1500, 8 heads
+// x 64 171 / 166 / -; 8 x 777 causal, 16 / 2 heads x 128 136 / 133 / 157; 16 of them
+// 240 / 240 / 318; 8 x 1500, 8 heads x 128 337 / 334 / 385.
+static bool attn_split_in_place(int batch, int tq, int hq) {
+    return (long long)batch * hq * ((tq + attn::QT - 1) / attn::QT) >= 768;
 }
 
-size_t attn_split_rows(int batch, int tq, int hq, int n_split) {
-    return (size_t)batch * hq * ((tq + attn::QT - 1) / attn::QT) * n_split * attn::QT;
-}
+// Partials of one launch: (query tile, head, chunk) slots of QT rows. The workspace
+// has this size whatever the call (134 MB of O at head_dim 128); a batch that needs more
+// slots runs in slices of whole items, which still fill the chip. It holds any one
+// item: with P <= kSplitTarget (query tile, head) pairs and chunks of at least 1 /
+// kSplitTarget of its tiles (a causal item's tiles are half its longest loop at least),
+// n <= 2 kSplitTarget / P + 1 chunks, 3 kSplitTarget slots. At 3 kSplitTarget the slices
+// of batches below the in-place line cost more than they hide (2 x 777 causal, 16 / 2
+// heads x 128: two slices 61 us, one launch 53; 32 x 64 queries over 1500 keys, 8
+// heads: 153, 132).
+constexpr size_t kSplitSlots = 4096;
+static_assert(kSplitSlots >= 3 * (size_t)kSplitTarget, "any item fits");
+size_t attn_split_rows() { return kSplitSlots * attn::QT; }
 
 hipError_t launch_flash_attn_split(hipStream_t s, int hd, const float* q, float q_scale, const void* kh, const void* kl,
                                    const void* vth, const void* vtl, float* out, int batch, int tq, int tkv, int t_pad,
-                                   int hq, int hkv, int causal, int q_off, const AttnSplit& sp) {
-    if ((long long)batch * sp.n_split > 65535 || sp.n_split < 2 || sp.chunk < 1) return hipErrorInvalidValue;
-    const bool seq = attn_split_in_place(hd, batch, tq, hq);
+                                   int hq, int hkv, int causal, int q_off, const AttnSplit& sp, const VkQOut* qo,
+                                   bool* fused) {
+    *fused = false;
+    if (sp.n_split < 2 || sp.chunk < 1) return hipErrorInvalidValue;
     FlashArgs a = {nullptr, nullptr, kh,     kl,      vth, vtl,
                    out,     tq,      tkv,    t_pad,   hq,  hkv,
                    causal,  q_off,   nullptr, q,      attn_q_scale(q_scale), VkQOut{},
                    attn_layout_rows(tkv, hkv, hd, t_pad)};
     a.sp = sp;
-    if (seq) {
-        hipLaunchKernelGGL((vk_flash_attn<64, 1, false, true>), dim3((tq + attn::QT - 1) / attn::QT, hq, batch), dim3(256), 0,
-                           s, (const uint4*)a.qh, (const uint4*)a.ql, (const uint4*)a.kh, (const uint4*)a.kl,
-                           (const uint4*)a.vth, (const uint4*)a.vtl, a.out, a.tq, a.tkv, a.t_pad, a.hq, a.hkv, a.causal,
-                           a.q_off, a.kv_index, a.qf, a.q_scale, a.qo, a.lay, a.sp);
-        return hipGetLastError();
+    const size_t slots = (size_t)((tq + attn::QT - 1) / attn::QT) * hq * sp.n_split;  // of one item
+    if (!sp.o || slots > kSplitSlots || attn_split_in_place(batch, tq, hq)) {
+        if (qo) a.qo = *qo;
+        if (qo && qo->afrag) {  // the activation pass runs in the kernel's epilogue
+            a.out = nullptr;
+            *fused = true;
+        }
+        return flash_any(s, hd, batch, KV_LO_F16, a, true);
     }
-    hipError_t e = flash_any(s, hd, batch, KV_LO_F16, a);
-    if (e != hipSuccess) return e;
-    if (hd == 64)
-        hipLaunchKernelGGL(vk_attn_combine<64>, dim3((tq + 15) / 16, hq, batch), dim3(256), 0, s, sp, out, tq, tkv, hq,
-                           causal, q_off);
-    else
-        hipLaunchKernelGGL(vk_attn_combine<128>, dim3((tq + 7) / 8, hq, batch), dim3(256), 0, s, sp, out, tq, tkv, hq,
-                           causal, q_off);
+    const int per = (int)std::min<size_t>(kSplitSlots / slots, (size_t)65535 / sp.n_split);  // items of a slice
+    for (int b = 0; b < batch; b += per) {
+        const int nb = std::min(per, batch - b);
+        const size_t ok = (size_t)b * tkv * hkv * hd * 2, ov = (size_t)b * hkv * hd * t_pad * 2;  // bytes
+        a.qf = q + (size_t)b * tq * hq * hd;
+        a.out = out + (size_t)b * tq * hq * hd;
+        a.kh = (const char*)kh + ok;
+        a.kl = (const char*)kl + ok;
+        a.vth = (const char*)vth + ov;
+        a.vtl = (const char*)vtl + ov;
+        const hipError_t e = flash_any(s, hd, nb, KV_LO_F16, a);
+        if (e != hipSuccess) return e;
+        if (hd == 64)
+            hipLaunchKernelGGL(vk_attn_combine<64>, dim3((tq + 15) / 16, hq, nb), dim3(256), 0, s, sp, a.out, tq, tkv,
+                               hq, causal, q_off);
+        else
+            hipLaunchKernelGGL(vk_attn_combine<128>, dim3((tq + 7) / 8, hq, nb), dim3(256), 0, s, sp, a.out, tq, tkv,
+                               hq, causal, q_off);
+    }
     return hipGetLastError();
 }
 

@@ -427,31 +427,31 @@ int check_attn(size_t batch, size_t tq, size_t tkv, size_t hq, size_t hkv, size_
 }
 
 // The key chunks of an attention call over several query rows (n_split = 1:
-// none), its partials' workspace in place. A capture cannot allocate: a call
-// whose partials no earlier call made room for records the undivided launch.
-int attn_split_for(vokra_hip_ctx* c, size_t batch, size_t tq, size_t tkv, size_t hq, size_t hd, int causal,
-                   size_t q_off, vk::AttnSplit* sp) {
+// none). Their partials' workspace has one size for every call and is allocated by
+// the first call that splits outside a capture; it is never replaced, so a captured
+// call's addresses stay good. Without it (a capture before, no memory) the chunks run
+// in place: same results.
+int attn_split_for(vokra_hip_ctx* c, size_t tq, size_t tkv, size_t hq, int causal, size_t q_off, vk::AttnSplit* sp) {
     *sp = vk::AttnSplit{nullptr, nullptr, 1, 0};
     if (q_off > (size_t)INT32_MAX / 2) return VOKRA_HIP_OK;
     int chunk = 0;
     const int n = vk::attn_key_splits((int)tq, (int)tkv, (int)hq, causal ? 1 : 0, (int)q_off, &chunk);
-    if (n <= 1 || batch * n > 65535) return VOKRA_HIP_OK;
-    const bool in_place = vk::attn_split_in_place((int)hd, (int)batch, (int)tq, (int)hq);
-    const size_t rows = in_place ? 0 : vk::attn_split_rows((int)batch, (int)tq, (int)hq, n);
-    if (c->at_po.cap < rows * hd * sizeof(float) || c->at_pml.cap < rows * sizeof(float2)) {
+    if (n <= 1) return VOKRA_HIP_OK;
+    const size_t rows = vk::attn_split_rows();
+    if (!c->at_pml.p) {
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
         VK_TRY(hipStreamIsCapturing(c->stream, &cs), "hipStreamIsCapturing");
-        if (cs != hipStreamCaptureStatusNone) return VOKRA_HIP_OK;
-        VK_TRY(c->at_po.ensure(rows * hd * sizeof(float)), "hipMalloc(attention partials)");
-        VK_TRY(c->at_pml.ensure(rows * sizeof(float2)), "hipMalloc(attention partials)");
+        if (cs == hipStreamCaptureStatusNone && (c->at_po.ensure(rows * 128 * sizeof(float)) != hipSuccess ||
+                                                 c->at_pml.ensure(rows * sizeof(float2)) != hipSuccess))
+            (void)hipGetLastError();  // no memory for it: clear the error
     }
-    *sp = vk::AttnSplit{(float*)c->at_po.p, (float2*)c->at_pml.p, n, chunk};
+    *sp = vk::AttnSplit{c->at_pml.p ? (float*)c->at_po.p : nullptr, (float2*)c->at_pml.p, n, chunk};
     return VOKRA_HIP_OK;
 }
 
 // With qo (a fused activation pass over the output rows), d_out is still
-// written when keep_out is set, when q is unaligned or when the keys split
-// (the pass then runs on it).
+// written when keep_out is set, when q is unaligned or when the keys split over
+// workgroups (the pass then runs on it).
 int run_attn(vokra_hip_ctx* c, size_t batch, size_t tq, size_t tkv, size_t hq, size_t hkv, size_t hd,
              const float* d_q, const float* d_k, const float* d_v, float scale, int causal, size_t q_off,
              float* d_out, const VkQOut* qo = nullptr, bool keep_out = true) {
@@ -488,14 +488,16 @@ int run_attn(vokra_hip_ctx* c, size_t batch, size_t tq, size_t tkv, size_t hq, s
     }
     vk::AttnSplit sp;
     if (q_in_kernel && !q7) {
-        int st = attn_split_for(c, batch, tq, tkv, hq, hd, causal, q_off, &sp);
+        int st = attn_split_for(c, tq, tkv, hq, causal, q_off, &sp);
         if (st) return st;
         if (sp.n_split > 1) {
+            bool fused = false;
             VK_TRY(vk::launch_flash_attn_split(c->stream, (int)hd, d_q, scale, c->at_kh.p, c->at_kl.p, c->at_vh.p,
                                                c->at_vl.p, d_out, (int)batch, (int)tq, (int)tkv, (int)t_pad, (int)hq,
-                                               (int)hkv, causal ? 1 : 0, (int)q_off, sp),
+                                               (int)hkv, causal ? 1 : 0, (int)q_off, sp, keep_out ? nullptr : qo,
+                                               &fused),
                    "launch(vk_flash_attn x key splits)");
-            if (qo)
+            if (qo && !fused)
                 VK_TRY(vk::launch_quantize_act_b32(c->stream, qo->pow2 != 0, d_out, (int)(batch * tq), qo->m_pad, qo->k,
                                                    qo->afrag, qo->ascale, qo->asum),
                        "launch(vk_quantize_act_b32)");
@@ -871,15 +873,17 @@ int attn_quantize_split(vokra_hip_ctx* c, size_t batch, size_t t, size_t h, size
         return fail(VOKRA_HIP_ERROR_INVALID_ARGUMENT, "attn: split operands need the fused activation pass");
     VK_TRY(set_dev(c), "hipSetDevice");
     vk::AttnSplit sp;
-    st = attn_split_for(c, batch, t, t, h, hd, 0, 0, &sp);
+    st = attn_split_for(c, t, t, h, 0, 0, &sp);
     if (st) return st;
     if (sp.n_split > 1) {  // as run_attn: the merged rows, then the activation pass
+        bool fused = false;
         VK_TRY(vk::launch_flash_attn_split(c->stream, (int)hd, d_q, scale, kh, kl, vth, vtl, d_out, (int)batch, (int)t,
-                                           (int)t, (int)t_pad, (int)h, (int)h, 0, 0, sp),
+                                           (int)t, (int)t_pad, (int)h, (int)h, 0, 0, sp, &qo, &fused),
                "launch(vk_flash_attn x key splits)");
-        VK_TRY(vk::launch_quantize_act_b32(c->stream, qo.pow2 != 0, d_out, (int)(batch * t), qo.m_pad, qo.k, qo.afrag,
-                                           qo.ascale, qo.asum),
-               "launch(vk_quantize_act_b32)");
+        if (!fused)
+            VK_TRY(vk::launch_quantize_act_b32(c->stream, qo.pow2 != 0, d_out, (int)(batch * t), qo.m_pad, qo.k,
+                                               qo.afrag, qo.ascale, qo.asum),
+                   "launch(vk_quantize_act_b32)");
     } else {
         VK_TRY(vk::launch_flash_attn_f32q(c->stream, (int)hd, d_q, scale, kh, kl, vth, vtl, nullptr, (int)batch, (int)t,
                                           (int)t, (int)t_pad, (int)h, (int)h, 0, 0, nullptr, vk::KV_LO_F16, &qo),

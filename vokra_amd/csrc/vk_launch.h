@@ -220,14 +220,19 @@ hipError_t launch_flash_attn(hipStream_t s, int hd, const void* qh, const void* 
 // kernel also quantizes O (rows b * tq + i, width hq * hd) into qo's
 // activation fragments, and out may be null.
 // How many chunks (1: none) the keys of one item's attention split into, and
-// the chunks' length in 64-key tiles; the workspace rows of such a launch.
+// the chunks' length in 64-key tiles.
 int attn_key_splits(int tq, int tkv, int hq, int causal, int q_off, int* chunk);
-size_t attn_split_rows(int batch, int tq, int hq, int n_split);
-bool attn_split_in_place(int hd, int batch, int tq, int hq);  // no partials: rows not needed
-// The flash launch over the chunks (f32 q, fp16 low parts) and their merge.
+// Rows of the partials' workspace (head_dim floats in sp.o, one pair in sp.ml each),
+// whatever the call.
+size_t attn_split_rows();
+// The flash launch over the chunks (f32 q, fp16 low parts) and their merge; a batch
+// that fills the chip, and one without a workspace (sp.o null), runs an item's chunks
+// in one workgroup per query tile instead, with the same results. *fused: the kernel
+// also ran qo's activation pass (out is then not written).
 hipError_t launch_flash_attn_split(hipStream_t s, int hd, const float* q, float q_scale, const void* kh, const void* kl,
                                    const void* vth, const void* vtl, float* out, int batch, int tq, int tkv, int t_pad,
-                                   int hq, int hkv, int causal, int q_off, const AttnSplit& sp);
+                                   int hq, int hkv, int causal, int q_off, const AttnSplit& sp, const VkQOut* qo,
+                                   bool* fused);
 hipError_t launch_flash_attn_f32q(hipStream_t s, int hd, const float* q, float q_scale, const void* kh, const void* kl,
                                   const void* vth, const void* vtl, float* out, int batch, int tq, int tkv, int t_pad,
                                   int hq, int hkv, int causal, int q_off, const int* kv_index = nullptr,
