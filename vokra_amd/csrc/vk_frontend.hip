@@ -96,7 +96,12 @@ __global__ __launch_bounds__(256) void vk_log_mel(const float* __restrict__ pcm,
     __shared__ float pw[FR][PW];
     __shared__ float2 tw[NFFT];  // W400^j
     __shared__ float red[4];
+    __shared__ int bad_lo[FR], bad_hi[FR];  // first and last bin of each frame whose power is not finite
     const int tid = threadIdx.x, b = blockIdx.y, t0 = blockIdx.x * FR;
+    if (tid < FR) {
+        bad_lo[tid] = NB;
+        bad_hi[tid] = -1;
+    }
     const float* clip = pcm + (size_t)b * n_samples;
     for (int i = tid; i < NFFT; i += 256) tw[i] = tw_g[i];
     for (int i = tid; i < FR * NC; i += 256) {
@@ -153,8 +158,13 @@ __global__ __launch_bounds__(256) void vk_log_mel(const float* __restrict__ pcm,
         const float2 e = make_float2(0.5f * (u.x + v.x), 0.5f * (u.y - v.y));
         const float2 o = fe_mul(make_float2(0.5f * (u.y + v.y), 0.5f * (v.x - u.x)), tw[k]);
         const float2 p = fe_add(e, o), m = fe_sub(e, o);
-        pw[f][k] = fmaf(p.x, p.x, p.y * p.y);
-        pw[f][NC - k] = fmaf(m.x, m.x, m.y * m.y);
+        const float pk = fmaf(p.x, p.x, p.y * p.y), pr = fmaf(m.x, m.x, m.y * m.y);
+        pw[f][k] = pk;
+        pw[f][NC - k] = pr;
+        if (!__builtin_isfinite(pk) || !__builtin_isfinite(pr)) {
+            atomicMin(&bad_lo[f], __builtin_isfinite(pk) ? NC - k : k);
+            atomicMax(&bad_hi[f], __builtin_isfinite(pr) ? k : NC - k);
+        }
     }
     __syncthreads();
     const int2* range = reinterpret_cast<const int2*>(fb);
@@ -166,6 +176,8 @@ __global__ __launch_bounds__(256) void vk_log_mel(const float* __restrict__ pcm,
         const int2 rg = range[m];
         float v = 0.0f;
         for (int k = rg.x; k < rg.y; ++k) v = fmaf(pw[f][k], w[(size_t)m * NB + k], v);
+        // the reference's sum runs over every bin: a zero weight makes NaN of a power that is not finite
+        if (bad_lo[f] < rg.x || bad_hi[f] >= rg.y) v = __builtin_nanf("");
         const float l = log10f(v > 1e-10f ? v : 1e-10f);
         out[((size_t)b * n_mels + m) * NFR + t] = l;
         mx = fmaxf(mx, l);
