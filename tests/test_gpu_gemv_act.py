@@ -59,3 +59,24 @@ def test_output_over_the_rows(ctx, oracle):
         ctx.gemm_q_f32_dev(w, 2, buf, At, d_b)
         got = buf.download(np.float32, 2 * n + 1024)[off // 4:off // 4 + 2 * n].reshape(2, n)
         assert np.array_equal(bits(got), bits(want))
+
+
+def test_one_row_makes_room_for_a_capture_of_more(oracle):
+    """A warm-up of one row, then a capture of eight, which take the activation pass of
+    their own: nothing is left to allocate, and every replay equals the eager call."""
+    ctx = hip.HipContext(0)
+    m, n, k = 8, 64, 1280
+    a, wq, bias = _gemm_case(oracle, hip.WDtype.Q4_0, m, n, k, seed=8)
+    w = hip.QWeight(ctx, hip.WDtype.Q4_0, n, k, wq)
+    d_a, d_b, d_o = hip.DeviceBuffer.from_array(ctx, a), hip.DeviceBuffer.from_array(ctx, bias), hip.DeviceBuffer(ctx, m * n * 4)
+    ctx.gemm_q_f32_dev(w, 1, d_a, d_o, d_b)
+    ctx.synchronize()
+    graph = ctx.capture(lambda: ctx.gemm_q_f32_dev(w, m, d_a, d_o, d_b))
+    want = np.ravel(oracle.gemm_qblock_i8(int(hip.WDtype.Q4_0), m, n, k, a, wq, bias))
+    for _ in range(3):
+        d_o.upload(np.zeros(m * n, np.float32))
+        graph.launch()
+        ctx.synchronize()
+        assert np.array_equal(bits(d_o.download(np.float32, m * n)), bits(want))
+    del graph
+    ctx.close()

@@ -399,6 +399,14 @@ int run_gemm(vokra_hip_ctx* c, const vokra_hip_qweight* w, size_t m, const float
     const bool apart = d_out + m * w->n <= d_a || d_a + m * w->k <= d_out;
     if (!w->kquant && act_quant != VOKRA_HIP_ACT_KQUANT && w->has_gemv && c->decode_kernel && m <= kGemvMaxM && apart &&
         vk::gemv_act_fits((int)m, (int)w->n, (int)w->nb)) {
+        // not used here, but a call of few rows makes room for as many as share its padding,
+        // so that a capture of more of them after it allocates nothing
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (c->act.frag.cap < round_up(m, vk::GEMM_TM) * w->k * 2) {
+            VK_TRY(hipStreamIsCapturing(c->stream, &cs), "hipStreamIsCapturing");
+            const int st = cs == hipStreamCaptureStatusNone ? qact_reserve(&c->act, m, w->k) : VOKRA_HIP_OK;
+            if (st) return st;
+        }
         const VkGemvLin lin = {(const uint4*)w->gq.p, (const uint2*)w->gsc.p, d_bias, d_out, {nullptr, 0}, (int)w->n};
         VK_TRY(vk::launch_gemv_qblock_act(c->stream, wd_kv_mode(w->wdtype), act_quant == VOKRA_HIP_ACT_POW2, d_a, lin,
                                           (int)m, (int)w->nb),
