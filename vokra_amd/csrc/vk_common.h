@@ -346,6 +346,14 @@ __device__ __forceinline__ uint32_t vk_lds_addr(const void* p) {
     return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
 }
 
+// Tile of workgroup L of a launch of `tiles`: the workgroups of one XCD (they go round
+// robin over the eight) take consecutive tiles, whatever the remainder.
+__device__ __forceinline__ int vk_xcd_tile(int L, int tiles) {
+    constexpr int N = 8;
+    const int per = tiles / N, rem = tiles - per * N, x = L % N;
+    return x * per + (x < rem ? x : rem) + L / N;
+}
+
 // Wait until at most N of this wave's vector-memory loads (the direct-to-LDS
 // loads above included) are in flight.
 template <int N>

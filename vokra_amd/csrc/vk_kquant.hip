@@ -667,7 +667,7 @@ __global__ __launch_bounds__(768) void vk_gemm_q4k(const uint4* __restrict__ afr
 // clocks per tile and group -> 71 at 2.2 GHz); m 1500, n 5120, k 1280 251 -> 101;
 // Q6_K 98 -> 60 and 292 -> 107.
 namespace kqt {
-constexpr int WAVES = 4, NS = 3, N_XCD = 8;  // waves per workgroup, ring stages
+constexpr int WAVES = 4, NS = 3;  // waves per workgroup, ring stages
 constexpr int THREADS = 64 * WAVES;
 template <int FMT>
 struct Fmt {
@@ -697,8 +697,7 @@ __global__ __launch_bounds__(kqt::THREADS, 2) void vk_gemm_kq_tiled(const uint4*
 
     // workgroup -> (column block, row block), column-major so that the row
     // blocks of one column block share its weights in one XCD's L2
-    const int tiles = (int)gridDim.x, L0 = blockIdx.x, per_xcd = tiles / N_XCD;
-    const int t = per_xcd * N_XCD == tiles ? (L0 % N_XCD) * per_xcd + L0 / N_XCD : L0;
+    const int t = vk_xcd_tile(blockIdx.x, gridDim.x);
     const int bx = t / tiles_m, mt0 = (t - bx * tiles_m) * WM;
     const int li = (set.count > 2 && bx >= set.tile0[2]) ? 2 : (set.count > 1 && bx >= set.tile0[1]) ? 1 : 0;
     const VkQ4kLin L = li == 2 ? set.l[2] : li == 1 ? set.l[1] : set.l[0];

@@ -15,6 +15,8 @@
 // 8*(l/16) .. 8*(l/16)+7. That is exactly the per-lane operand of
 // v_mfma_f32_16x16x32_bf16, so a wave loads a fragment with one coalesced
 // 16-byte-per-lane read. Tiles are ordered [row_tile][block][lane][8].
+#include <algorithm>
+
 #include "vk_common.h"
 
 namespace vk {
@@ -695,8 +697,7 @@ __global__ __launch_bounds__(gemm::THREADS, 2) void vk_gemm_qblock_deep(
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
 
-    const int tiles_lin = tiles_m * tiles_n, tiles = tiles_lin * n_lin, L = blockIdx.x, per_xcd = tiles / gemm::N_XCD;
-    const int tt = (per_xcd * gemm::N_XCD == tiles) ? (L % gemm::N_XCD) * per_xcd + L / gemm::N_XCD : L;
+    const int tiles_lin = tiles_m * tiles_n, tt = vk_xcd_tile(blockIdx.x, tiles_lin * n_lin);
     const int li = tt / tiles_lin, t = tt - li * tiles_lin;
     const int ntile = t / tiles_m, mtile = t - ntile * tiles_m;
     const int mt0 = mtile * 2 * MT, nt0 = ntile * 2 * NT;  // first fragment tiles
@@ -959,7 +960,9 @@ constexpr int kGemmSmallTileBelow = 384;  // 128 x 128 tiles per launch
 // split outputs; the fused activation pass stays with the kernel above): 32 x 32
 // workgroup tiles up to kDeepTiles, fewer when K is long, where each extra
 // round of workgroups costs a whole K loop; then, for long K, 64 x 64 tiles
-// while one resident round (3 workgroups on each of 256 CUs) holds them.
+// while one resident round (3 workgroups on each of 256 CUs) holds them, and fewer the
+// shorter K is (4 groups per quant block): their gain is the K loop's latency, and a
+// CU with three of them shares its matrix cores as the other kernel's does.
 // Measured, us, vk_gemm_qblock / 32 x 32 / 64 x 64 (m, n, k): 960 tiles (187,
 // 1280, 5120) 42.1 / 15.6 / 35.3; 1520 (300, 1280, 1280) 13.0 / 7.1 / 12.8; 3024
 // (1000, 768, 768) 9.1 / 6.8 / 9.8; 3040 (600, 1280, 5120) 43.4 / 28.1 / 35.9;
@@ -967,7 +970,11 @@ constexpr int kGemmSmallTileBelow = 384;  // 128 x 128 tiles per launch
 // 17.8; 4512 (1500, 768, 3072) 31.0 / 32.0 / 27.4; 6080 (300, 5120, 1280) 16.7 /
 // 19.0 / 15.6; 7520 (1500, 1280, 5120) 55 / 90 / 45; 8000 (4000, 512, 2048) 23.3 /
 // 42.4 / 26.3; 12032, 768 groups (1500, 2048, 5632) 79 / 155 / 71; 15040, 940
-// groups (3000, 1280, 5120) 91 / 178 / 111.
+// groups (3000, 1280, 5120) 91 / 178 / 111. Whole calls, vk_gemm_qblock / 64 x 64, by
+// groups: k 3072: 288 39.8 / 36.0, 564 49.2 / 52.5, 756 61.0 / 65.2; k 4096: 384 49.1 /
+// 44.3, 512 51.4 / 49.5, 640 62.6 / 62.7, 752 71.5 / 73.8; k 5120: 540 72.9 / 68.6, 640
+// 76.4 / 76.7, 760 88.3 / 89.8; k 5632: 608 77.9 / 72.2, 704 83.0 / 79.0; k 6144: 576
+// 81.5 / 78.8.
 constexpr size_t kDeepTiles = 4200, kDeepTilesLongK = 3200, kDeepWideGroups = 768;
 constexpr int kDeepWideBlocks = 96;  // k >= 3072
 
@@ -998,7 +1005,7 @@ hipError_t launch_gemm_qblock_multi(hipStream_t s, bool pow2, const uint4* afrag
         if (pow2) VK_GDEEP(true, 1, 1, 4);
         VK_GDEEP(false, 1, 1, 4);
     }
-    if (!qout && t16 >= 1 && nb >= kDeepWideBlocks && w64 <= kDeepWideGroups) {
+    if (!qout && t16 >= 1 && nb >= kDeepWideBlocks && w64 <= std::min(kDeepWideGroups, (size_t)4 * nb)) {
         if (pow2) VK_GDEEP(true, 2, 2, 2);
         VK_GDEEP(false, 2, 2, 2);
     }
