@@ -17,9 +17,10 @@ def ctx():
 
 
 # the smallest such vocabulary and one row less; 64- and 128-row workgroups with one
-# row left; every number of column tiles, and more streams than a workgroup holds
+# row left; every number of column tiles, and more streams than a workgroup holds;
+# row distances whose workgroups start along k (4 KiB multiples)
 @pytest.mark.parametrize("n,v,d", [(3, 30719, 128), (3, 30720, 128), (16, 30785, 256), (17, 32769, 128), (33, 49153, 128),
-                                   (64, 49153, 384), (65, 30721, 128)])
+                                   (64, 49153, 384), (65, 30721, 128), (33, 30721, 1024), (2, 30720, 2048)])
 def test_wide_logits(ctx, oracle, n, v, d):
     print(f"[case] wide logits n={n} v={v} d={d}", flush=True)
     g = np.random.default_rng(n + v + d)

@@ -538,8 +538,8 @@ __global__ __launch_bounds__(64 * lg::WAVES) void vk_logits_argmax(const float* 
 // 128-byte lines), four steps ahead. The streams' fragments are shared: split by the
 // workgroup one step ahead into LDS, one barrier per step.
 //
-// Bound: memory, 4 bytes per weight: 64 streams, 51866 x 1280 (265 MB) 144
-// -> 86 us (52 at the rate of a copy, 30 of products and splits on each SIMD).
+// Bound: memory, 4 bytes per weight: 64 streams, 51866 x 1280 (265 MB) 149
+// -> 83 us (52 at the rate of a copy, 30 of products and splits on each SIMD).
 // Error against 64 bits, relative to the largest logit: 1.6e-7, the f32 kernel's 5.2e-7.
 namespace lx3 {
 constexpr int WAVES = 4, RING = 4;  // RING: steps of vocabulary rows in flight
@@ -588,17 +588,28 @@ __global__ __launch_bounds__(64 * lx3::WAVES, 2) void vk_logits_argmax_x3(const 
     char* xw = reinterpret_cast<char*>(&lx[0][0][stage ? ss >> 4 : 0][(ss & 15) + 16 * (sk >> 3)]) + 2 * (sk & 7);
     constexpr int PART = NCT * 64 * 16, BUF = 3 * PART;  // bytes
     const int nk = d / 32;  // a multiple of RING
+    // Where this workgroup's walk over k starts. Rows a multiple of 4 KiB apart lie on the
+    // same memory channels, and workgroups that all start at k = 0 meet there: those of an
+    // XCD (every eighth) then start one ring after the other. One stream / 64, us, from 0 and
+    // rotated: 51865 x 1024 54.2 / 69.4 -> 46.4 / 65.7, 32000 x 2048 55.3 / 82.9 -> 48.0 / 82.1;
+    // other distances lose by it: 51865 x 512 27.0 / 42.0 -> 29.0 / 43.0, 30720 x 1280 33.8 /
+    // 54.0 -> 34.9 / 53.9.
+    const int rot = d % 1024 == 0 ? (int)((blockIdx.x >> 3) % (unsigned)(nk / RING)) * RING : 0;
+    auto step_at = [&](int ks) {  // step ks of the walk; past the end: the last one again, unused
+        const int t = min(ks, nk - 1) + rot;
+        return t < nk ? t : t - nk;
+    };
     vk_f32x8 er[RING][J];
     XVec xr[RING];
     auto load_e = [&](int u, int ks) {
-        const int at = 8 * min(ks, nk - 1);  // past the end: the last step again, unused
+        const int at = 8 * step_at(ks);
 #pragma unroll
         for (int j = 0; j < J; ++j) {
             const float4 a = ep[j][at], b = ep[j][at + 1];
             er[u][j] = (vk_f32x8){a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
         }
     };
-    auto load_x = [&](int u, int ks) { __builtin_memcpy(&xr[u], __builtin_assume_aligned(xp + 32 * min(ks, nk - 1), XW == 2 ? 8 : 16), 4 * XW); };
+    auto load_x = [&](int u, int ks) { __builtin_memcpy(&xr[u], __builtin_assume_aligned(xp + 32 * step_at(ks), XW == 2 ? 8 : 16), 4 * XW); };
     auto store_x = [&](int u, int buf) {
         const VkBf16x3<XW> t = vk_split_bf16x3<XW>(xr[u]);
         if (!stage) return;
@@ -927,9 +938,11 @@ static int go_logits_wide(hipStream_t s, const float* x, const float* emb, float
 // Vocabularies from which the three-part kernel runs, whatever the number of streams (a
 // stream's logits do not depend on its batch): its k loop is one chain per workgroup,
 // four times as long as the f32 kernel's, and needs about two workgroups per CU to hide
-// it. f32 / three-part, us: 51866 x 1280: 64 streams 144 / 86, 17 71 / 58, 16 65 / 54, 8
-// 58 / 53, 1 50 / 54; 40000 x 1280, 64 streams 93 / 66; 32000 x 2048 115 / 84; 20000 x
-// 1280: 64 streams 57 / 50, 16 29 / 31; 5000 x 512, 64 streams 14.5 / 19.
+// it. f32 / three-part, us, one stream, four and 64: 51866 x 1280 65.9 / 60.3, 71.5 / 61.4,
+// 149 / 83; 51865 x 1024 48.5 / 46.8, 52.8 / 48.0, 115 / 66; 51865 x 512 27.7 / 27.2, 30.5 /
+// 28.3, 70 / 42; 32000 x 2048 53.7 / 48.4, 58.1 / 48.8, 121 / 81; 30720 x 1280 41.1 / 33.9,
+// 44.1 / 34.7, 89 / 55. Below, fewer streams lose: 20000 x 1280 57 / 50 with 64, 29 / 31 with
+// 16; 5000 x 512, 64 streams 14.5 / 19.
 constexpr int kLogitsWideFrom = 30720;
 
 hipError_t launch_logits_argmax(hipStream_t s, const float* x, const float* emb, float* logits, float2* part,
