@@ -24,7 +24,7 @@ constexpr int T = 64, KC = 16, PAD = 4;
 
 template <bool BT>
 __global__ __launch_bounds__(256) void vk_gemm_f32(const float* __restrict__ a, const float* __restrict__ b,
-                                                   const float* __restrict__ bias, VkEpi epi, float* out, int m,
+                                                   const float* __restrict__ bias, float* out, int m,
                                                    int n, int k) {
     using namespace g32;
     __shared__ float as[KC][T + PAD];
@@ -91,7 +91,7 @@ __global__ __launch_bounds__(256) void vk_gemm_f32(const float* __restrict__ a, 
                 const int gm = m0 + wr + 16 * i + 4 * (lane >> 4) + r, gn = n0 + wc + 16 * j + (lane & 15);
                 if (gm < m && gn < n) {
                     const size_t o = (size_t)gm * n + gn;
-                    out[o] = vk_epi_apply(bias ? bias[gn] + acc[i][j][r] : acc[i][j][r], epi, o);
+                    out[o] = bias ? bias[gn] + acc[i][j][r] : acc[i][j][r];
                 }
             }
 }
@@ -109,7 +109,7 @@ constexpr int TM = 128, TN = 128, KC = 16, NS = 3, N_XCD = 8;
 
 template <bool BT>
 __global__ __launch_bounds__(256, 2) void vk_gemm_f32_tiled(const float* __restrict__ a, const float* __restrict__ b,
-                                                            const float* __restrict__ bias, VkEpi epi, float* out,
+                                                            const float* __restrict__ bias, float* out,
                                                             int m, int n, int k) {
     using namespace g32f;
     __shared__ __align__(16) float la[NS][TM * KC];  // [row][k], 8 KiB per stage
@@ -201,7 +201,7 @@ __global__ __launch_bounds__(256, 2) void vk_gemm_f32_tiled(const float* __restr
                 const int gm = m0 + wm * 64 + 16 * i + 4 * g + r, gn = n0 + wn * 64 + 16 * j + l16;
                 if (gm < m && gn < n) {
                     const size_t o = (size_t)gm * n + gn;
-                    out[o] = vk_epi_apply(bias ? bias[gn] + acc[i][j][r] : acc[i][j][r], epi, o);
+                    out[o] = bias ? bias[gn] + acc[i][j][r] : acc[i][j][r];
                 }
             }
 }
@@ -807,7 +807,7 @@ __global__ __launch_bounds__(256) void vk_argmax_slices(const float* __restrict_
 namespace vk {
 
 hipError_t launch_gemm_f32(hipStream_t s, bool b_trans, const float* a, const float* b, const float* bias,
-                           float* out, int m, int n, int k, VkEpi epi) {
+                           float* out, int m, int n, int k) {
     if (m == 0 || n == 0) return hipSuccess;
     // the tiled kernel: whole 16-wide K stages (at least two), 16-byte aligned
     // rows, and for B [k, n] whole column quads
@@ -815,16 +815,16 @@ hipError_t launch_gemm_f32(hipStream_t s, bool b_trans, const float* a, const fl
     if (k % g32f::KC == 0 && k >= 2 * g32f::KC && aligned && (b_trans || n % 4 == 0)) {
         const unsigned tiles = (unsigned)(((m + g32f::TM - 1) / g32f::TM) * ((n + g32f::TN - 1) / g32f::TN));
         if (b_trans)
-            hipLaunchKernelGGL(vk_gemm_f32_tiled<true>, dim3(tiles), dim3(256), 0, s, a, b, bias, epi, out, m, n, k);
+            hipLaunchKernelGGL(vk_gemm_f32_tiled<true>, dim3(tiles), dim3(256), 0, s, a, b, bias, out, m, n, k);
         else
-            hipLaunchKernelGGL(vk_gemm_f32_tiled<false>, dim3(tiles), dim3(256), 0, s, a, b, bias, epi, out, m, n, k);
+            hipLaunchKernelGGL(vk_gemm_f32_tiled<false>, dim3(tiles), dim3(256), 0, s, a, b, bias, out, m, n, k);
         return hipGetLastError();
     }
     const dim3 grid((n + g32::T - 1) / g32::T, (m + g32::T - 1) / g32::T);
     if (b_trans)
-        hipLaunchKernelGGL(vk_gemm_f32<true>, grid, dim3(256), 0, s, a, b, bias, epi, out, m, n, k);
+        hipLaunchKernelGGL(vk_gemm_f32<true>, grid, dim3(256), 0, s, a, b, bias, out, m, n, k);
     else
-        hipLaunchKernelGGL(vk_gemm_f32<false>, grid, dim3(256), 0, s, a, b, bias, epi, out, m, n, k);
+        hipLaunchKernelGGL(vk_gemm_f32<false>, grid, dim3(256), 0, s, a, b, bias, out, m, n, k);
     return hipGetLastError();
 }
 

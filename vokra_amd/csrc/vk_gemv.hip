@@ -145,9 +145,6 @@ struct GemvSet {
     VkGemvLin lin[3];
 };
 
-// DEV: the linears come from a device array (any count, one per grid z) rather
-// than the kernel arguments.
-//
 // ACT: the activations come as f32 rows x [m][32 nb] and every workgroup quantizes
 // its tile's rows itself, into LDS, with the arithmetic of the activation pass, while
 // its weights are on their way: one launch instead of two. Eight lanes hold a block,
@@ -421,6 +418,8 @@ __device__ __forceinline__ void gemv_w_tile(const uint4* __restrict__ afrag, con
     }
 }
 
+// DEV: the linears come from a device array (any count, one per grid z) rather
+// than the kernel arguments.
 template <int MODE, bool POW2, bool DEV>
 __global__ __launch_bounds__(64) void vk_gemv_qblock_w(
     const uint4* __restrict__ afrag, const float* __restrict__ ascale, const float* __restrict__ asum,

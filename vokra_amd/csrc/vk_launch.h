@@ -304,8 +304,7 @@ hipError_t launch_kv_alloc_layers(hipStream_t s, const KvView& v, int layer0, in
 
 namespace vk {
 hipError_t launch_gemm_f32(hipStream_t s, bool b_trans, const float* a, const float* b, const float* bias,
-                           float* out, int m, int n, int k,
-                           VkEpi epi = {nullptr, 0});
+                           float* out, int m, int n, int k);
 hipError_t launch_gemv_f32(hipStream_t s, const float* a, const float* x, const float* bias, float* out, int m,
                            int k);
 hipError_t launch_softmax_f32(hipStream_t s, const float* in, float* out, int rows, int cols);
