@@ -44,6 +44,28 @@ def test_append_batches_lockstep(ctx, oracle, H, hd, n):
                        for a, b in zip(got, want))
 
 
+def test_append_rows_off_16_bytes(ctx):
+    """A small batch whose rows start off 16 bytes takes the two launches: same cache."""
+    H, hd, n = 2, 64, 5
+    g = np.random.default_rng(9)
+    streams, times = np.arange(n, dtype=np.int32) % 3, np.arange(n, dtype=np.int32) * 3
+    k, v = (g.standard_normal((n, H * hd)).astype(np.float32) for _ in range(2))
+    a, b = (ctx.kv_cache(1, H, hd, 3, 32, 4) for _ in range(2))
+    a.append(0, streams, times, k, v)
+    d_s, d_t = (hip.DeviceBuffer.from_array(ctx, x) for x in (streams, times))
+    rows = [hip.DeviceBuffer.from_array(ctx, np.concatenate([np.full(1, 9.0, np.float32), np.ravel(x)])) for x in (k, v)]
+
+    class Off:
+        def __init__(self, buf):
+            self.ptr = type(buf.ptr)(buf.ptr.value + 4)
+    b.append_dev(0, n, d_s, d_t, *(Off(r) for r in rows))
+    b.status()
+    assert a.pages() == b.pages()
+    for i in range(n):
+        x, y = (c.read(0, int(times[i]), int(streams[i])) for c in (a, b))
+        assert np.array_equal(x[0], y[0]) and np.array_equal(x[1], y[1])
+
+
 @pytest.mark.parametrize("bad", [0, 5, 7])
 def test_append_stops_at_the_first_invalid_item(ctx, bad):
     kv = ctx.kv_cache(1, 2, 64, 4, 32, 4)
