@@ -144,26 +144,19 @@ hipError_t launch_swiglu_quantize_g16(hipStream_t s, const float* g, const float
 }  // namespace vk
 
 namespace vk {
-// The conv stem (vk_stem.hip): weights as scaled fp16 hi / lo [out][3][channels]
-// (channels padded to stem_channels), and a batch's workspaces: hi / lo rows of
-// the log-mel [clip][n_frames + 2][stem_channels(n_mels)] and of the first
-// convolution's output [clip][n_frames + 2][d], and stem_scalars(batch) floats.
+// The conv stem (vk_stem.hip): packed weights (stem_weight_halves 16-bit values each),
+// and a batch's workspaces: the parts of the log-mel and of the first convolution's
+// output (stem_mel_halves, stem_hidden_halves). d a multiple of 32.
 struct StemW {
-    const void *w1hi, *w1lo, *w2hi, *w2lo;
-    int e1, e2;  // their scales' exponents
+    const void *w1, *w2;
     const float *b1, *b2, *pos;
-    float l1max, bmax;  // largest row L1 norm of conv1's weights, largest |conv1 bias|
 };
-struct StemBufs {
-    void *ahi, *alo, *hhi, *hlo;
-    float* scal;
-};
-inline int stem_channels(int c) { return (c + 31) / 32 * 32; }
-size_t stem_scalars(size_t batch);
-int stem_weight_exponent(const float* w, size_t n);
-hipError_t launch_stem_pack(hipStream_t s, const float* w, int out, int c, int cp, int e, void* hi, void* lo);
-hipError_t launch_stem(hipStream_t s, const float* mel, int batch, int nm, int nf, int nc, int d, const StemW& w,
-                       const StemBufs& b, float* out);
+size_t stem_weight_halves(int out, int c);
+size_t stem_mel_halves(size_t batch, int nm, int nf);
+size_t stem_hidden_halves(size_t batch, int d, int nf);
+hipError_t launch_stem_pack(hipStream_t s, const float* w, int out, int c, void* wp);
+hipError_t launch_stem(hipStream_t s, const float* mel, size_t batch, int nm, int nf, int nc, int d, const StemW& w,
+                       void* mel_parts, void* hidden_parts, float* out);
 }  // namespace vk
 
 namespace vk {

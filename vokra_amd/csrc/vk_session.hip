@@ -144,12 +144,10 @@ struct vokra_hip_encoder {
     std::vector<EncLayer> layers;
     DBuf lnpg, lnpb, h, x, q, k, v, attn, f;
     vokra_hip_qact_t *qa_d = nullptr, *qa_f = nullptr;
-    // conv stem (optional): fp16 hi / lo weights with their scales, positional
-    // embedding, the two convolutions' input rows
+    // conv stem (optional): packed weights, biases, positional embedding, the two
+    // convolutions' input parts
     size_t n_mels = 0, n_frames = 0, n_ctx = 0, stem_batch = 0;
-    DBuf c1hi, c1lo, c1b, c2hi, c2lo, c2b, pos, st_a, st_h, st_scal;
-    int c1e = 0, c2e = 0;
-    float c1_l1max = 0.0f, c1_bmax = 0.0f;
+    DBuf c1w, c1b, c2w, c2b, pos, parts;
     // attention V^T as fp16 hi / lo [batch][d / hd][hd][t_pad] (the v split
     // pass's output; k's hi / lo, written by the q/k/v GEMM, take k's own
     // buffer)
@@ -160,9 +158,8 @@ struct vokra_hip_encoder {
             for (DBuf* b : {&L.ln1g, &L.ln1b, &L.ln2g, &L.ln2b}) b->release(ctx);
             for (QLin* w : {&L.q, &L.k, &L.v, &L.o, &L.fc1, &L.fc2}) w->release(ctx);
         }
-        for (DBuf* b : {&lnpg, &lnpb, &h, &x, &q, &k, &v, &attn, &f, &c1hi, &c1lo, &c1b, &c2hi, &c2lo, &c2b, &pos,
-                        &st_a, &st_h, &st_scal,
-                        &vt_hi, &vt_lo})
+        for (DBuf* b : {&lnpg, &lnpb, &h, &x, &q, &k, &v, &attn, &f, &c1w, &c1b, &c2w, &c2b, &pos, &parts, &vt_hi,
+                        &vt_lo})
             b->release(ctx);
         vt_cap = 0;
         vokra_hip_qact_free(qa_d);
@@ -299,39 +296,28 @@ int enc_forward(vokra_hip_encoder* e, size_t batch, size_t frames, const float* 
 // encoder.rs:58-104) into d_x [batch, n_ctx, d] (vk_stem.hip).
 int enc_stem(vokra_hip_encoder* e, size_t batch, const float* d_mel, float* d_x) {
     vokra_hip_ctx_t* c = e->ctx;
-    const size_t d = e->d, nf = e->n_frames, mp = (size_t)vk::stem_channels((int)e->n_mels);
-    const size_t na = batch * (nf + 2) * mp, nh = batch * (nf + 2) * d;  // values of each half
-    if (batch > e->stem_batch) {  // workspaces grow with the largest batch seen
-        for (DBuf* b : {&e->st_a, &e->st_h, &e->st_scal}) b->release(c);
+    const int d = (int)e->d, nm = (int)e->n_mels, nf = (int)e->n_frames;
+    const size_t mel = vk::stem_mel_halves(batch, nm, nf);
+    if (batch > e->stem_batch) {  // the workspace grows with the largest batch seen
+        e->parts.release(c);
         e->stem_batch = 0;
-        SS_TRY(e->st_a.alloc(c, 2 * na * sizeof(uint16_t)));
-        SS_TRY(e->st_h.alloc(c, 2 * nh * sizeof(uint16_t)));
-        SS_TRY(e->st_scal.alloc(c, vk::stem_scalars(batch) * sizeof(float)));
+        SS_TRY(e->parts.alloc(c, (mel + vk::stem_hidden_halves(batch, d, nf)) * sizeof(uint16_t)));
         e->stem_batch = batch;
     }
-    const vk::StemW w = {e->c1hi.p, e->c1lo.p, e->c2hi.p, e->c2lo.p, e->c1e, e->c2e, e->c1b.f(), e->c2b.f(),
-                         e->pos.f(), e->c1_l1max, e->c1_bmax};
-    const vk::StemBufs b = {e->st_a.p, (uint16_t*)e->st_a.p + na, e->st_h.p, (uint16_t*)e->st_h.p + nh,
-                            e->st_scal.f()};
-    SS_HIP(vk::launch_stem(vk::ctx_stream(c), d_mel, (int)batch, (int)e->n_mels, (int)nf, (int)e->n_ctx, (int)d, w, b,
-                           d_x),
+    uint16_t* parts = (uint16_t*)e->parts.p;  // the log-mel's, then the first convolution's
+    const vk::StemW w = {e->c1w.p, e->c2w.p, e->c1b.f(), e->c2b.f(), e->pos.f()};
+    SS_HIP(vk::launch_stem(vk::ctx_stream(c), d_mel, batch, nm, nf, (int)e->n_ctx, d, w, parts, parts + mel, d_x),
            "launch(vk_stem)");
     return VOKRA_HIP_OK;
 }
 
-// One convolution's weights [out][channels][3] on the host -> scaled fp16 hi /
-// lo [out][3][channels padded] on the device.
-int stem_upload(vokra_hip_ctx_t* c, const float* w, size_t out, size_t ch, DBuf& hi, DBuf& lo, int* e,
-                const char* what) {
-    const size_t cp = (size_t)vk::stem_channels((int)ch);
+// One convolution's weights [out][channels][3] on the host -> packed on the device.
+int stem_upload(vokra_hip_ctx_t* c, const float* w, size_t out, size_t ch, DBuf& packed, const char* what) {
     DBuf f32;
     int st = upload_vec(c, f32, w, out * ch * 3, what);
-    *e = vk::stem_weight_exponent(w, out * ch * 3);
-    if (!st) st = hi.alloc(c, out * 3 * cp * sizeof(uint16_t));
-    if (!st) st = lo.alloc(c, out * 3 * cp * sizeof(uint16_t));
+    if (!st) st = packed.alloc(c, vk::stem_weight_halves((int)out, (int)ch) * sizeof(uint16_t));
     if (!st) {
-        const hipError_t he =
-            vk::launch_stem_pack(vk::ctx_stream(c), f32.f(), (int)out, (int)ch, (int)cp, *e, hi.p, lo.p);
+        const hipError_t he = vk::launch_stem_pack(vk::ctx_stream(c), f32.f(), (int)out, (int)ch, packed.p);
         if (he != hipSuccess)
             st = vk::ctx_fail(VOKRA_HIP_ERROR_BACKEND_UNAVAILABLE, "%s: %s", what, hipGetErrorString(he));
     }
@@ -561,23 +547,12 @@ int vokra_hip_encoder_set_stem(vokra_hip_ctx_t* c, vokra_hip_encoder_t* e, size_
     if (n_mels == 0 || n_mels > 1024 || n_frames < 2 || n_frames > 65536)
         return vk::ctx_fail(VOKRA_HIP_ERROR_INVALID_ARGUMENT, "encoder_set_stem: n_mels 1..1024, n_frames 2..65536");
     const size_t d = e->d, n_ctx = (n_frames + 2 - 3) / 2 + 1;  // conv_out_len(n_frames, 3, 2, 1)
-    for (DBuf* b : {&e->c1hi, &e->c1lo, &e->c1b, &e->c2hi, &e->c2lo, &e->c2b, &e->pos, &e->st_a, &e->st_h, &e->st_scal})
-        b->release(c);
-    e->stem_batch = 0;  // workspaces depend on the stem's shape
+    for (DBuf* b : {&e->c1w, &e->c1b, &e->c2w, &e->c2b, &e->pos, &e->parts}) b->release(c);
+    e->stem_batch = 0;  // the workspace depends on the stem's shape
     e->n_ctx = 0;       // no stem until this one is whole
-    SS_TRY(stem_upload(c, conv1_w, d, n_mels, e->c1hi, e->c1lo, &e->c1e, "encoder_set_stem: conv1_w"));
+    SS_TRY(stem_upload(c, conv1_w, d, n_mels, e->c1w, "encoder_set_stem: conv1_w"));
     SS_TRY(upload_vec(c, e->c1b, conv1_b, d, "encoder_set_stem: conv1_b"));
-    SS_TRY(stem_upload(c, conv2_w, d, d, e->c2hi, e->c2lo, &e->c2e, "encoder_set_stem: conv2_w"));
-    // bound of the first convolution's output per unit of input (finite weights)
-    double l1 = 0.0, bm = 0.0;
-    for (size_t o = 0; o < d; ++o) {
-        double s = 0.0;
-        for (size_t i = 0; i < n_mels * 3; ++i) s += std::isfinite(conv1_w[o * n_mels * 3 + i]) ? std::fabs((double)conv1_w[o * n_mels * 3 + i]) : 0.0;
-        l1 = std::max(l1, s);
-        bm = std::max(bm, std::isfinite(conv1_b[o]) ? std::fabs((double)conv1_b[o]) : 0.0);
-    }
-    e->c1_l1max = (float)std::min(l1, 3.0e38);
-    e->c1_bmax = (float)bm;
+    SS_TRY(stem_upload(c, conv2_w, d, d, e->c2w, "encoder_set_stem: conv2_w"));
     SS_TRY(upload_vec(c, e->c2b, conv2_b, d, "encoder_set_stem: conv2_b"));
     SS_TRY(upload_vec(c, e->pos, pos_emb, n_ctx * d, "encoder_set_stem: pos_emb"));
     e->n_mels = n_mels;
