@@ -133,7 +133,7 @@ def test_stem_infinities_and_the_largest_finite_value(ctx):
 
 
 def test_stem_of_many_short_clips(ctx):
-    """More clips than a grid has rows in y and z."""
+    """Clip and row counts past 16 bits; each clip as alone."""
     g = np.random.default_rng(7)
     n, d = 65537, 64
     W = weights(g, 1, d, 0.3)

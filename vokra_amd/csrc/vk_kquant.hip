@@ -651,8 +651,8 @@ __global__ __launch_bounds__(768) void vk_gemm_q4k(const uint4* __restrict__ afr
 // trip of every term through LDS and the adding waves).
 //
 // Bound: the combine's five VALU operations per output and 16-wide group. With
-// two or more waves resident a SIMD issues a plain f32 multiply or add every 2.3
-// clocks (4.5 with one; DPP, integer and three-operand forms 4.2 always) and a
+// two or more waves resident a SIMD issues an f32 multiply, add or FMA every 2.3 to 2.9
+// clocks (4.9 to 5.8 with one; DPP forms, and_or, shifts and conversions 4.2) and a
 // 16x16x16 MFMA every 16, and the two do not overlap: a 16 x 16 tile and group
 // is 20 of the former (46 clocks), one MFMA and the unpacking (~16). So:
 //  * the accumulator input -128 * gsum (see vk_gemm_q4k) depends on the rows
